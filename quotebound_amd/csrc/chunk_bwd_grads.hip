@@ -8,13 +8,17 @@
 // pass) and the chunk's tile (T, P, exp G, D, beta from prep), the state rows are streamed in blocks of 32:
 //   KS = K S0^T, R = V - diag(exp G) KS, Delta = T (diag(beta) R), KdS = K dS^T,
 //   dDelta = P^T dY + D KdS, dR' = T^T dDelta, dR = diag(beta) dR'     (D = diag(exp(G_63 - G)))
-//   dP^T += Delta dY^T, dT^T += (diag(beta) R) dDelta^T, dbeta += rowsum(R * dR'),
+//   dP^T += Delta dY^T, dA -= dR' Delta^T, dbeta += rowsum(R * dR'),
 //   dQ_inter += dY S0, dK += -diag(exp G) dR S0 + D Delta dS
 // then, once per value head, the 64 x 64 part:
 //   dQ += diag(exp G) dQ_inter + (dP * M) K,  dK += (dP * M)^T Q + (dKK + dKK^T) K
-//   dA = -T^T dT T^T,  dKK = strict_lower(diag(beta) dA * E)
+//   dKK = strict_lower(diag(beta) dA * E)
 //   dbeta_j += sum_m dA_jm E_jm (K K^T)_jm,  dG from every exp(.) factor, dg = reverse cumsum
-// (dbeta's first term, sum_i dTb_ij T_ij with Tb = T diag(beta), equals sum_r R_jr (T^T dDelta)_jr.)
+// (dbeta's first term, sum_i dTb_ij T_ij with Tb = T diag(beta), equals sum_r R_jr (T^T dDelta)_jr. dA is the
+// adjoint of T = (I + A)^-1, -T^T dT T^T with dT = dDelta (diag(beta) R)^T: the two outer factors meet dDelta and R
+// as T^T dDelta = dR' and T diag(beta) R = Delta, which the row blocks have at hand. Forming dA there from dT in three
+// products with T, two barriers more, took the kernel 159.8 us against 153.1 at B = 1, T = 4096, 16 and 32 heads,
+// 227.3 against 219.9 with 48 value heads.)
 // (tests/chunk_math.py restates these equations and checks them against the oracle.) Wave w owns positions
 // 16 (w % 4) .. + 15 and, within each product, the half w / 4 of the other index (state rows of a 32-row block,
 // key-position tiles, or 64 of the 128 columns). MFMA with split float32 operands as in the forward. Each
@@ -43,20 +47,19 @@ constexpr int kLP = 80;   // [32][64]
 constexpr int kLT = 80;   // T, P [64][64]
 constexpr int oS0h = 0, oS0l = oS0h + 32 * kLS, odSh = oS0l + 32 * kLS, odSl = odSh + 32 * kLS;
 constexpr int odYh = odSl + 32 * kLS, odYl = odYh + kC * kLY;
-constexpr int oRh = odYl + kC * kLY, oRl = oRh + 32 * kLP;        // diag(beta) R, R = V - diag(exp G) K S0^T
+constexpr int oRh = odYl + kC * kLY, oRl = oRh + 32 * kLP;        // diag(beta) R, R = V - diag(exp G) K S0^T; dR'
 constexpr int oDh = oRl + 32 * kLP, oDl = oDh + 32 * kLP;         // Delta
 constexpr int oDDh = oDl + 32 * kLP, oDDl = oDDh + 32 * kLP;      // D Delta
 constexpr int odDh = oDDl + 32 * kLP, odDl = odDh + 32 * kLP;     // dDelta
 constexpr int oGdRh = odDl + 32 * kLP, oGdRl = oGdRh + 32 * kLP;  // -diag(exp G) dR
 constexpr int kLoopBytes = (oGdRl + 32 * kLP) * 2;
-// End-phase region (aliases the block-loop region), bf16 element offsets: Q rows, then P * M, Z^T (Z = dT T^T) and
-// dKK^T, each as hi and lo 64 x 64 matrices; then float32 per-position partial sums. (K rows stay in their own array
-// for the whole block and T in TL for the whole value head; dT reuses the P array.)
+// End-phase region (aliases the block-loop region), bf16 element offsets: Q rows, then P * M and dKK^T, each as hi
+// and lo 64 x 64 matrices; then float32 per-position partial sums. (K rows stay in their own array for the whole
+// block.)
 constexpr int kLK = 144;
 constexpr int eQb = 0;
 constexpr int eMh = eQb + kC * kLK, eMl = eMh + kC * kLT;  // P * M
-constexpr int eZh = eMl + kC * kLT, eZl = eZh + kC * kLT;
-constexpr int eKh = eZl + kC * kLT, eKl = eKh + kC * kLT;
+constexpr int eKh = eMl + kC * kLT, eKl = eKh + kC * kLT;
 constexpr int eF = (eKl + kC * kLT) / 2;  // first float32 offset
 constexpr int eX2r = eF, eX2c = eX2r + 2 * kC, edbA = eX2c + 4 * kC;
 constexpr int ex1c = edbA + 2 * kC, etq = ex1c + 4 * kC;
@@ -64,7 +67,7 @@ constexpr int kEndBytes = (etq + 2 * kC) * 4;
 constexpr int kSmemBytes = kLoopBytes > kEndBytes ? kLoopBytes : kEndBytes;
 
 // The key tile (16 positions j) that accumulator mi of the wave at position tile pw, half hw holds in dP^T and
-// dT^T. Only tiles m <= pw carry work. For each pw the two halves together hold all four tiles; positions 0..31
+// dA. Only tiles m <= pw carry work. For each pw the two halves together hold all four tiles; positions 0..31
 // alternate the tiles between halves so each half works on one of the tiles 0..pw, positions 32..63 split them in
 // halves. The busiest wave of the phase that accumulates them then runs 5 products in place of 6.
 __device__ __forceinline__ int key_tile(int pw, int hw, int mi) { return pw < 2 ? hw + 2 * mi : 2 * hw + mi; }
@@ -194,13 +197,13 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
 #pragma unroll
     for (int t = 0; t < 4; ++t) dQ[t] = zero4(), dK[t] = zero4();
     // (K K^T)[p][m], rows p = 16 pw + 4g + jj, columns m = 16 key_tile(pw, hw, mi) + li; zero above tile pw. The same
-    // for every value head of the group: formed in the item's first one's end phase.
+    // for every value head of the group: formed at the start of the item's first one.
     f32x4 kk[2];
 
     for (int e = cur.e0; e < cur.e0 + cur.ne; ++e) {
       const int hv = hk * grp + e;
-      // The head whose tile and first block the end phase reads ahead, in pieces at the starts of E2, E3 and E4
-      // (beside their products, so that no phase issues them all): the next in the group, the next item's first,
+      // The head whose tile and first block the end phase reads ahead, in two pieces in E1 and at the
+      // start of E2 (all of them in E2, whose products the waves then reach late, measured 154.3 against 153.1 us): the next in the group, the next item's first,
       // or, for the block's last item, this head again (those reads are unused; they keep every path's loads the
       // same, so the compiler's waits stay exact).
       Item nx = cur;
@@ -220,13 +223,29 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
         *reinterpret_cast<bf16x8*>(PL[0] + lt8) = ti.tp[2];
         *reinterpret_cast<bf16x8*>(PL[1] + lt8) = ti.tp[3];
       }
-      f32x4 dPt[2], dTt[2], dQi[4];  // dPt, dTt: key tiles m = key_tile(pw, hw, mi); lane -> column i = ip, rows j
+      // Key tiles m = key_tile(pw, hw, mi): dPt lane -> column i = ip, rows j; nA = -dA laid out as kk.
+      f32x4 dPt[2], nA[2], dQi[4];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) dPt[t] = zero4(), dTt[t] = zero4();
+      for (int t = 0; t < 2; ++t) dPt[t] = zero4(), nA[t] = zero4();
 #pragma unroll
       for (int t = 0; t < 4; ++t) dQi[t] = zero4();
       float gpart[4] = {0.f, 0.f, 0.f, 0.f}, hD[4] = {0.f, 0.f, 0.f, 0.f}, bpart[4] = {0.f, 0.f, 0.f, 0.f}, sds = 0.f;
       __syncthreads();
+      if (e == cur.e0) {
+        int lt = tid;
+        asm volatile("" : "+v"(lt));
+        const int g = (lt >> 4) & 3, li = lt & 15, pw = (lt >> 6) & 3, hw = lt >> 8, ip = 16 * pw + li;
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi) {
+          const int m = key_tile(pw, hw, mi);
+          kk[mi] = zero4();
+          if (m <= pw) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+              kk[mi] = mma(kk[mi], lds8(Kres + swz(ip, 32 * s + 8 * g, kLK)), lds8(Kres + swz(16 * m + li, 32 * s + 8 * g, kLK)));
+          }
+        }
+      }
 
       // The end phase's inputs (Q rows, as bf16 bits), loaded during the value head's last block into the registers
       // the next block's reads would use: thread -> Q row e / 16, columns 8 (e % 16) .. + 7 for e = tid, tid + 512.
@@ -345,8 +364,8 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
         __syncthreads();
         if constexpr (more) load_dy_v(nb, cur, hv, r0 + 32, lt);
 
-        // Phase 3: dR = diag(beta) T^T dDelta (and dbeta's T part, R * (T^T dDelta) summed over the rows); dP^T +=
-        // Delta dY^T and dT^T += (diag(beta) R) dDelta^T over this half's key tiles.
+        // Phase 3: dR' = T^T dDelta, dR = diag(beta) dR' (and dbeta's T part, R * dR' summed over the rows), dR' into
+        // R's place (R's last readers were phase 2's); dP^T += Delta dY^T over this half's key tiles.
         {
           f32x4 dr = zero4();
 #pragma unroll
@@ -359,6 +378,7 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
               dr = mma3(dr, TtA, Split8{lds8(sb + odDh + at), lds8(sb + odDl + at)});
             }
           }
+          put4(sb + oRh, sb + oRl, swz(r, i0, kLP), dr);
           float gdr[4];
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {
@@ -369,28 +389,31 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
           }
           put4(sb + oGdRh, sb + oGdRl, swz(r, i0, kLP), gdr[0], gdr[1], gdr[2], gdr[3]);
         }
-        {
-          // dDelta[i][r] of the wave's positions as B (k = r, n = i).
-          const Split8 BdD{lds_tr8s(sb + odDh + 16 * pw, kLP, lt), lds_tr8s(sb + odDl + 16 * pw, kLP, lt)};
 #pragma unroll
-          for (int mi = 0; mi < 2; ++mi) {
-            const int m = key_tile(pw, hw, mi);
-            if (m <= pw) {
-              // Delta and diag(beta) R rows j of key tile m as A (m = j, k = r).
-              const Split8 AD{lds_tr8s(sb + oDh + 16 * m, kLP, lt), lds_tr8s(sb + oDl + 16 * m, kLP, lt)};
-              if constexpr (kExactDy)
-                dPt[mi] = mma2(dPt[mi], AD, dYo.hi);
-              else
-                dPt[mi] = mma3(dPt[mi], AD, dYo);
-              const Split8 AR{lds_tr8s(sb + oRh + 16 * m, kLP, lt), lds_tr8s(sb + oRl + 16 * m, kLP, lt)};
-              dTt[mi] = mma3(dTt[mi], AR, BdD);
-            }
+        for (int mi = 0; mi < 2; ++mi) {
+          const int m = key_tile(pw, hw, mi);
+          if (m <= pw) {
+            // Delta rows j of key tile m as A (m = j, k = r).
+            const Split8 AD{lds_tr8s(sb + oDh + 16 * m, kLP, lt), lds_tr8s(sb + oDl + 16 * m, kLP, lt)};
+            if constexpr (kExactDy)
+              dPt[mi] = mma2(dPt[mi], AD, dYo.hi);
+            else
+              dPt[mi] = mma3(dPt[mi], AD, dYo);
           }
         }
         __syncthreads();
 
-        // Phase 4: dQ_inter += dY S0; dK += -diag(exp G) dR S0 + D Delta dS (columns of this half).
+        // Phase 4: -dA += dR' Delta^T over this half's key tiles; dQ_inter += dY S0; dK += -diag(exp G) dR S0 +
+        // D Delta dS (columns of this half).
         {
+          // dR'[p][r] of the wave's positions as A (k = r), Delta[m][r] as B (k = r, n = m).
+          const Split8 AdR{lds_tr8s(sb + oRh + 16 * pw, kLP, lt), lds_tr8s(sb + oRl + 16 * pw, kLP, lt)};
+#pragma unroll
+          for (int mi = 0; mi < 2; ++mi) {
+            const int m = key_tile(pw, hw, mi);
+            if (m <= pw)
+              nA[mi] = mma3(nA[mi], AdR, Split8{lds_tr8s(sb + oDh + 16 * m, kLP, lt), lds_tr8s(sb + oDl + 16 * m, kLP, lt)});
+          }
           const Split8 AGdR{lds_tr8s(sb + oGdRh + 16 * pw, kLP, lt), lds_tr8s(sb + oGdRl + 16 * pw, kLP, lt)};
           const Split8 ADD{lds_tr8s(sb + oDDh + 16 * pw, kLP, lt), lds_tr8s(sb + oDDl + 16 * pw, kLP, lt)};
 #pragma unroll
@@ -429,10 +452,11 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
       }
       __syncthreads();
 
-      // E1: Q rows into the end-phase region. Per lane, at i = ip and j = 16 key_tile(pw, hw, mi) + 4g + jj (dP and
-      // dT masked to j <= i): the row and column sums of dP * P (the P factor's part of dG), P * M with
-      // M_ij = exp(G_i - G_j) over P's entries into the end-phase region, and dT, both as hi and lo, dT in place of P
-      // (each lane rewrites only the P entries it has just read).
+      // E1: Q rows into the end-phase region. Per lane, at i = ip and j = 16 key_tile(pw, hw, mi) + 4g + jj (dP masked
+      // to j <= i): the row and column sums of dP * P (the P factor's part of dG), and P * M with M_ij =
+      // exp(G_i - G_j) over P's entries into the end-phase region. Then at rows p = i0 + jj and columns
+      // m = 16 key_tile(pw, hw, mi) + li, as kk: dA's products with E = exp(G_p - G_m) and K K^T, the A part of dbeta
+      // (row sums) and of dG (row and column sums), and dKK = diag(beta) (dA * E), stored as dKK^T.
       {
         {
 #pragma unroll
@@ -441,6 +465,9 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
             *reinterpret_cast<uint4*>(sb + eQb + swz(e >> 4, (e & 15) * 8, kLK)) = __builtin_bit_cast(uint4, nb.ys[q2]);
           }
         }
+        // The next head's tile and first S0 rows (ti was staged at this head's start, nb.xs at its last block's).
+        load_tile(ti, nx, nhv, lt);
+        load_rows(nb.xs, a.ckpt, nx, nhv, 0, lt);
         // Row sums (over j) add up over g here and over hw in dG; column sums (over i) over li here and over pw in dG.
         float prow = 0.f;
         const float gi = Gf[ip];
@@ -450,7 +477,7 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
           const uint2 ph = *reinterpret_cast<const uint2*>(PL[0] + at);
           const uint2 pl = *reinterpret_cast<const uint2*>(PL[1] + at);
           const uint32_t hw4[2] = {ph.x, ph.y}, lw4[2] = {pl.x, pl.y};
-          float pm[4], db[4];
+          float pm[4];
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {
             const int j = j0 + jj;
@@ -464,113 +491,21 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
             x2c[pw][j] = col;
             // Where j > i, dp is zero and the exponent positive: clamped at 0 to keep the product finite.
             pm[jj] = dp * __expf(fminf(gi - Gf[j], 0.f));
-            db[jj] = j <= ip ? dTt[mi][jj] : 0.f;
           }
           put4(sb + eMh, sb + eMl, at, pm[0], pm[1], pm[2], pm[3]);
-          put4(PL[0], PL[1], at, db[0], db[1], db[2], db[3]);
         }
         prow = swap32_sum(swap16_sum(prow));
         x2r[hw][ip] = prow;  // the same bits in the four lane groups
-      }
-      __syncthreads();
-
-      {  // the next head's tile (ti was staged at this head's start)
-        int lq = tid;
-        asm volatile("" : "+v"(lq));
-        load_tile(ti, nx, nhv, lq);
-      }
-      // E2: dQ += diag(exp G) dQ_inter and its dG term; K K^T (the first value head only, kept in registers);
-      // dQ += (P * M) K; dK += (P * M)^T Q; Z = dT T^T, stored as Z^T.
-      {
-        float tq[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj) {
-            const int i = i0 + jj, c = 16 * (4 * hw + t) + li;
-            tq[jj] += (float)sb[eQb + swz(i, c, kLK)] * dQi[t][jj];
-            dQ[t][jj] += gam[i] * dQi[t][jj];
-          }
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const float v = sum16(tq[jj]);
-          tpos[hw][i0 + jj] = v;
-        }
-        if (e == cur.e0) {
-#pragma unroll
-          for (int mi = 0; mi < 2; ++mi) {
-            const int m = key_tile(pw, hw, mi);
-            kk[mi] = zero4();
-            if (m <= pw) {
-#pragma unroll
-              for (int s = 0; s < 4; ++s)
-                kk[mi] = mma(kk[mi], lds8(Kres + swz(ip, 32 * s + 8 * g, kLK)), lds8(Kres + swz(16 * m + li, 32 * s + 8 * g, kLK)));
-            }
-          }
-        }
-        // P * M is zero above the diagonal: rows i < 32 end at column 31, and columns j >= 32 start at row 32.
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          if (s == 0 || pw >= 2) {
-            const int at = swz(ip, 32 * s + 8 * g, kLT);
-            const Split8 Apm{lds8(sb + eMh + at), lds8(sb + eMl + at)};  // (P * M) rows i = ip, k = j
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-              dQ[t] = mma2(dQ[t], Apm, lds_tr8s(Kres + 32 * s * kLK + 16 * (4 * hw + t), kLK, lt));
-          }
-          if (s == 1 || pw < 2) {
-            const Split8 Apmt{lds_tr8s(sb + eMh + 32 * s * kLT + 16 * pw, kLT, lt),
-                              lds_tr8s(sb + eMl + 32 * s * kLT + 16 * pw, kLT, lt)};  // (P * M)^T rows j = ip, k = i
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-              dK[t] = mma2(dK[t], Apmt, lds_tr8s(sb + eQb + 32 * s * kLK + 16 * (4 * hw + t), kLK, lt));
-          }
-        }
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi) {
-          const int mr = 16 * (2 * hw + mi) + li;  // this lane's column m of Z
-          f32x4 z = zero4();
-#pragma unroll
-          for (int s = 0; s < 2; ++s) {
-            const int aa = swz(ip, 32 * s + 8 * g, kLT), ab = swz(mr, 32 * s + 8 * g, kLT);
-            z = mma3(z, Split8{lds8(PL[0] + aa), lds8(PL[1] + aa)}, Split8{lds8(TL[0] + ab), lds8(TL[1] + ab)});
-          }
-          put4(sb + eZh, sb + eZl, swz(mr, i0, kLT), z[0], z[1], z[2], z[3]);
-        }
-      }
-      __syncthreads();
-
-      load_rows(nb.xs, a.ckpt, nx, nhv, 0, lt);  // the next head's first S0 rows (nb.xs went to LDS in E1)
-      // E3: dA = -T^T Z below the diagonal (rows p = i0 + jj, columns m = 16 key_tile(pw, hw, mi) + li, as kk), and at
-      // once its products with E = exp(G_p - G_m) and K K^T: the A part of dbeta (row sums), of dG (row and column
-      // sums), and dKK = diag(beta) (dA * E), stored as dKK^T.
-      {
-        // Only tiles mt <= pw are kept (mcol < p), and T^T rows p >= 32 are zero below column 32.
-        Split8 AT[2];  // T^T rows p = ip, k = i
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-          AT[s] = Split8{lds_tr8s(TL[0] + 32 * s * kLT + 16 * pw, kLT, lt),
-                         lds_tr8s(TL[1] + 32 * s * kLT + 16 * pw, kLT, lt)};
         float rowp[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int mi = 0; mi < 2; ++mi) {
-          const int mt = key_tile(pw, hw, mi), mcol = 16 * mt + li;
-          f32x4 da = zero4();
-          if (mt <= pw) {
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-              if (s == 1 || pw < 2) {
-                const int ab = swz(mcol, 32 * s + 8 * g, kLT);
-                da = mma3(da, AT[s], Split8{lds8(sb + eZh + ab), lds8(sb + eZl + ab)});
-              }
-            }
-          }
+          const int mcol = 16 * key_tile(pw, hw, mi) + li;
           float colp = 0.f, kkt[4];
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {
             const int pr = i0 + jj;
             const float e = __expf(fminf(Gf[pr] - Gf[mcol], 0.f));  // finite everywhere; used where mcol < pr
-            const float dae = mcol < pr ? -da[jj] * e : 0.f;           // dA_pm E_pm
+            const float dae = mcol < pr ? -nA[mi][jj] * e : 0.f;       // dA_pm E_pm
             const float prod = dae * kk[mi][jj];
             rowp[jj] += prod;
             colp += bet[pr] * prod;
@@ -588,26 +523,63 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
       }
       __syncthreads();
 
-      load_rows(nb.ys, a.dsend, nx, nhv, 0, lt);  // and its first dS rows, dy and v
-      load_dy_v(nb, nx, nhv, 0, lt);
-      // E4: dK += (dKK + dKK^T) K for rows j = ip, this half's columns: dKK rows j through the transposing read of
-      // dKK^T, dKK^T rows j directly.
+      {  // the next head's first dS rows, dy and v (nb.ys went to LDS in E1)
+        int lq = tid;
+        asm volatile("" : "+v"(lq));
+        load_rows(nb.ys, a.dsend, nx, nhv, 0, lq);
+        load_dy_v(nb, nx, nhv, 0, lq);
+      }
+      // E2: dQ += diag(exp G) dQ_inter and its dG term; dQ += (P * M) K; dK += (P * M)^T Q; dK += (dKK + dKK^T) K for
+      // rows j = ip, this half's columns: dKK rows j through the transposing read of dKK^T, dKK^T rows j directly.
+      {
+        float tq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int at = swz(ip, 32 * s + 8 * g, kLT);
-        const Split8 A1{lds_tr8s(sb + eKh + 32 * s * kLT + 16 * pw, kLT, lt), lds_tr8s(sb + eKl + 32 * s * kLT + 16 * pw, kLT, lt)};
-        const Split8 A2{lds8(sb + eKh + at), lds8(sb + eKl + at)};
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const bf16x8 B = lds_tr8s(Kres + 32 * s * kLK + 16 * (4 * hw + t), kLK, lt);
-          // dKK is strictly lower: dKK[j][i] needs i < j, dKK[i][j] needs i > j.
-          if (s == 0 || pw >= 2) dK[t] = mma2(dK[t], A1, B);
-          if (s == 1 || pw < 2) dK[t] = mma2(dK[t], A2, B);
+          for (int jj = 0; jj < 4; ++jj) {
+            const int i = i0 + jj, c = 16 * (4 * hw + t) + li;
+            tq[jj] += (float)sb[eQb + swz(i, c, kLK)] * dQi[t][jj];
+            dQ[t][jj] += gam[i] * dQi[t][jj];
+          }
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const float v = sum16(tq[jj]);
+          tpos[hw][i0 + jj] = v;
+        }
+        // P * M is zero above the diagonal: rows i < 32 end at column 31, and columns j >= 32 start at row 32. dKK is
+        // strictly lower: dKK[j][i] needs i < j, dKK[i][j] needs i > j.
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          bf16x8 B[4];  // K rows 32 s .., this half's columns
+#pragma unroll
+          for (int t = 0; t < 4; ++t) B[t] = lds_tr8s(Kres + 32 * s * kLK + 16 * (4 * hw + t), kLK, lt);
+          const int at = swz(ip, 32 * s + 8 * g, kLT);
+          if (s == 0 || pw >= 2) {
+            const Split8 Apm{lds8(sb + eMh + at), lds8(sb + eMl + at)};  // (P * M) rows i = ip, k = j
+            const Split8 A1{lds_tr8s(sb + eKh + 32 * s * kLT + 16 * pw, kLT, lt), lds_tr8s(sb + eKl + 32 * s * kLT + 16 * pw, kLT, lt)};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              dQ[t] = mma2(dQ[t], Apm, B[t]);
+              dK[t] = mma2(dK[t], A1, B[t]);
+            }
+          }
+          if (s == 1 || pw < 2) {
+            const Split8 Apmt{lds_tr8s(sb + eMh + 32 * s * kLT + 16 * pw, kLT, lt),
+                              lds_tr8s(sb + eMl + 32 * s * kLT + 16 * pw, kLT, lt)};  // (P * M)^T rows j = ip, k = i
+            const Split8 A2{lds8(sb + eKh + at), lds8(sb + eKl + at)};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              dK[t] = mma2(dK[t], Apmt, lds_tr8s(sb + eQb + 32 * s * kLK + 16 * (4 * hw + t), kLK, lt));
+              dK[t] = mma2(dK[t], A2, B[t]);
+            }
+          }
         }
       }
-      // E5 (one wave): dG per position, dg = its reverse cumulative sum (a suffix scan over the wave), and dbeta.
+      __syncthreads();
+      // E3 (one wave): dG per position, dg = its reverse cumulative sum, and dbeta. Lane l takes position 63 - l, so
+      // that the sum runs up the lanes, as a DPP scan.
       if (tid < kC) {
-        const int t = tid;
+        const int t = kC - 1 - tid;
         const float hs = hpos[0][t] + hpos[1][t];
         float hsum = sum16(hs);
         hsum = swap32_sum(swap16_sum(hsum));
@@ -619,11 +591,7 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
                   (x1cp[0][t] + x1cp[1][t] + x1cp[2][t] + x1cp[3][t]) + x2r[0][t] + x2r[1][t] -
                   (x2c[0][t] + x2c[1][t] + x2c[2][t] + x2c[3][t]);
         if (t == kC - 1) v += hsum + gam[kC - 1] * sds_all;
-#pragma unroll
-        for (int off = 1; off < kC; off <<= 1) {
-          const float u = __shfl_down(v, off);
-          if (t + off < kC) v += u;
-        }
+        v = wave_prefix_sum(v);
         if constexpr (kFused) {
           const int64_t g0 = tok * a.Hv + hv;
           const uint32_t gi = uint32_t(t * a.Hv);
@@ -665,7 +633,7 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
       continue;
     }
     if constexpr (kFused) {
-      // dq, dk rounded to bf16 into rows [64][128] in the end phase's bytes (E5's reads of them done), then the
+      // dq, dk rounded to bf16 into rows [64][128] in the end phase's bytes (E3's reads of them done), then the
       // normalisation's backward row by row, 16 lanes of 8 elements per row as in the separate pass: the raw rows,
       // and the results, through buffer resources that end at the chunk's last row.
       __syncthreads();

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace qbgdn {
 
 constexpr int kChunk = 64;     // checkpoint stride, the reference's kChunk (src/delta_grad.cpp:11)
@@ -148,6 +150,24 @@ __device__ __forceinline__ void sum32_pair(float& a, float& b) {
   const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   a = __uint_as_float(t[0]);
   b = __uint_as_float(t[1]);
+}
+
+// The inclusive prefix sum over the wave's 64 lanes: within each row of 16 lanes by row_shr 1, 2, 4, 8 (lanes without
+// a source add zero), then row 0's total into row 1 and row 2's into row 3 (row_bcast 15), then the first two rows'
+// into the last two (row_bcast 31). VALU only, where six __shfl steps are LDS round trips.
+__device__ __forceinline__ float wave_prefix_sum(float x) {
+  const auto add = [&x](auto ctrl, auto rows) {
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, decltype(rows)::value,
+                                                    0xf, false));
+  };
+  using std::integral_constant;
+  add(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});
+  add(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
+  return x;
 }
 
 // Blocks are dispatched round-robin over the MI355X's 8 XCDs (block id runs on XCD id % 8), each with its own
