@@ -4,8 +4,10 @@ There is no fallback: if the library is missing or fails to load, every call rai
 """
 from __future__ import annotations
 
+import collections
 import ctypes
 import os
+import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libqb_gdn.so")
@@ -101,6 +103,52 @@ def make_desc(B, T, Hk, Hv, Dk, Dv, *, dtype=BF16, g_is_log=True, design=CHUNKED
     return d, keep
 
 
+class Plan:
+    """What a call of one shape and set of options needs besides its tensors: the checked descriptor and the sizes that
+    follow from it. Never written to once made, so threads and streams share it."""
+
+    __slots__ = ("desc", "ref", "keep", "workspace", "ckpt_floats")
+
+    def __init__(self, desc, keep, workspace, ckpt_floats=0):
+        self.desc, self.keep, self.ref = desc, keep, ctypes.byref(desc)
+        self.workspace, self.ckpt_floats = max(workspace, 1), max(ckpt_floats, 1)
+
+
+# Plans by their values (shape, options, sequence bounds and the device, whose size enters a workspace's), the least
+# recently used ones dropped. Forming one (a descriptor, two checks, two sizes) takes about 9 us of a call's host time,
+# as long as the one-token kernel runs; a program calls the same few shapes again and again.
+_PLANS_KEPT = 256
+_plans = collections.OrderedDict()
+_plans_lock = threading.Lock()
+
+
+def plan(key, make):
+    """The plan of `key`; make() forms it and raises where there is none."""
+    with _plans_lock:
+        p = _plans.get(key)
+        if p is not None:
+            _plans.move_to_end(key)
+            return p
+    p = make()
+    with _plans_lock:
+        _plans[key] = p
+        while len(_plans) > _PLANS_KEPT:
+            _plans.popitem(last=False)
+    return p
+
+
+_local = threading.local()
+
+
+def _err():
+    """This thread's buffer for a failing call's reason."""
+    try:
+        return _local.err
+    except AttributeError:
+        _local.err = ctypes.create_string_buffer(512)
+        return _local.err
+
+
 def validate(desc) -> str | None:
     """None when the library accepts desc, else its reason."""
     err = ctypes.create_string_buffer(512)
@@ -145,20 +193,12 @@ def fwd_rows(desc, q, k, v, g, beta, s0, y, row_states, stream) -> None:
 
 
 def fwd(desc, q, k, v, g, beta, s0, y, s_out, ckpt, workspace, stream) -> None:
-    """Pointers are ints (device addresses) or None; raises RuntimeError with the library's reason on failure."""
-    err = ctypes.create_string_buffer(512)
-    rc = load().qb_gdn_fwd(ctypes.byref(desc), q, k, v, g, beta, s0, y, s_out, ckpt, workspace, stream, err,
-                           len(err))
-    if rc != 0:
-        raise RuntimeError(err.value.decode())
+    """desc, here and below, is a descriptor or a Plan. Pointers are ints (device addresses) or None; raises RuntimeError with the library's reason on failure."""
+    _call(load().qb_gdn_fwd, desc, q, k, v, g, beta, s0, y, s_out, ckpt, workspace, stream)
 
 
 def bwd(desc, q, k, v, g, beta, ckpt, dy, ds_out, dq, dk, dv, dg, dbeta, ds0, workspace, stream) -> None:
-    err = ctypes.create_string_buffer(512)
-    rc = load().qb_gdn_bwd(ctypes.byref(desc), q, k, v, g, beta, ckpt, dy, ds_out, dq, dk, dv, dg, dbeta, ds0,
-                           workspace, stream, err, len(err))
-    if rc != 0:
-        raise RuntimeError(err.value.decode())
+    _call(load().qb_gdn_bwd, desc, q, k, v, g, beta, ckpt, dy, ds_out, dq, dk, dv, dg, dbeta, ds0, workspace, stream)
 
 
 def bwd_static(desc, q, k, v, g, beta, ckpt, dy, ds_out, dq, dk, dv, dg, dbeta, ds0, stream) -> None:
@@ -174,8 +214,8 @@ def neighbours_workspace_bytes(desc) -> int:
 
 
 def _call(fn, desc, *args) -> None:
-    err = ctypes.create_string_buffer(512)
-    if fn(ctypes.byref(desc), *args, err, len(err)) != 0:
+    err = _err()
+    if fn(desc.ref if type(desc) is Plan else ctypes.byref(desc), *args, err, 512) != 0:
         raise RuntimeError(err.value.decode())
 
 

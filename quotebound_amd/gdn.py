@@ -29,40 +29,56 @@ def _dev_ptr(t):
 
 
 def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _io_dtype(*ts):
     """bf16 when every activation is bf16, else float32 (the reference computes in float32 either way)."""
-    return torch.bfloat16 if all(t.dtype == torch.bfloat16 for t in ts) else torch.float32
+    for t in ts:
+        if t.dtype != torch.bfloat16:
+            return torch.float32
+    return torch.bfloat16
+
+
+def _as(t, dtype):
+    """t in dtype, contiguous."""
+    return t if t.dtype == dtype and t.is_contiguous() else t.to(dtype).contiguous()
 
 
 def _prep(q, k, v, g, beta, dtype):
     if not q.is_cuda:
         raise RuntimeError("gated delta: tensors must be on a HIP device (there is no CPU path)")
-    c = lambda t: t.to(dtype).contiguous()  # noqa: E731
-    return c(q), c(k), c(v), g.to(torch.float32).contiguous(), c(beta)
+    return _as(q, dtype), _as(k, dtype), _as(v, dtype), _as(g, torch.float32), _as(beta, dtype)
 
 
-def _desc(q, v, dtype, g_is_log, design, cu_seqlens, out_f32):
+def _plan(q, v, dtype, g_is_log, design, cu_seqlens, out_f32):
+    """The call's plan; raises with the library's reason where it refuses the call."""
     B, T, Hk, Dk = q.shape
     Hv, Dv = v.shape[2], v.shape[3]
-    make = lambda d: _lib.make_desc(B, T, Hk, Hv, Dk, Dv,  # noqa: E731
-                                    dtype=_lib.BF16 if dtype == torch.bfloat16 else _lib.F32, g_is_log=g_is_log,
-                                    design=d, cu_seqlens=cu_seqlens, out_f32=out_f32)
-    if design is None:
-        longest = T if cu_seqlens is None else max(int(b) - int(a) for a, b in zip(cu_seqlens[:-1], cu_seqlens[1:]))
-        if longest > SHORT_T:
-            desc, keep = make(_lib.CHUNKED)
-            if not _lib.validate(desc):
-                return desc, keep
-        design = _lib.RECURRENT
-    return make(design)
+    bf16 = dtype == torch.bfloat16
+    cu = None if cu_seqlens is None else tuple([int(x) for x in cu_seqlens])
+    out_f32, g_is_log = bool(out_f32), bool(g_is_log)
+
+    def make():
+        desc = lambda d: _lib.make_desc(B, T, Hk, Hv, Dk, Dv, dtype=_lib.BF16 if bf16 else _lib.F32,  # noqa: E731
+                                        g_is_log=g_is_log, design=d, cu_seqlens=cu, out_f32=out_f32)
+        if design is not None:
+            pair = desc(design)
+        else:
+            longest = T if cu is None else max([y - x for x, y in zip(cu[:-1], cu[1:])])
+            pair = desc(_lib.CHUNKED) if longest > SHORT_T else None
+            if pair is None or _lib.validate(pair[0]):
+                pair = desc(_lib.RECURRENT)
+        why = _lib.validate(pair[0])
+        if why:
+            raise RuntimeError(why)
+        return _lib.Plan(*pair, _lib.workspace_bytes(pair[0]), _lib.ckpt_bytes(pair[0]) // 4)
+
+    return _lib.plan((torch._C._cuda_getDevice(), B, T, Hk, Hv, Dk, Dv, bf16, g_is_log, design, out_f32, cu), make)
 
 
-def _workspace(desc, device):
-    n = _lib.workspace_bytes(desc)
-    return torch.empty(max(n, 1), dtype=torch.uint8, device=device)
+def _workspace(plan, device):
+    return torch.empty(plan.workspace, dtype=torch.uint8, device=device)
 
 
 def forward(q, k, v, g, beta, state=None, *, log_decay=False, design=DEFAULT_DESIGN, cu_seqlens=None,
@@ -71,24 +87,20 @@ def forward(q, k, v, g, beta, state=None, *, log_decay=False, design=DEFAULT_DES
     y is in the inputs' dtype, or float32 with out_f32."""
     dtype = _io_dtype(q, k, v, beta)
     q, k, v, g, beta = _prep(q, k, v, g, beta, dtype)
-    desc, keep = _desc(q, v, dtype, log_decay, design, cu_seqlens, out_f32)
+    plan = _plan(q, v, dtype, log_decay, design, cu_seqlens, out_f32)
     odt = torch.float32 if out_f32 else dtype
-    why = _lib.validate(desc)
-    if why:
-        raise RuntimeError(why)
     N = q.shape[0] if cu_seqlens is None else len(cu_seqlens) - 1
     dev = q.device
     Hv, Dv, Dk = v.shape[2], v.shape[3], q.shape[3]
-    s0 = None if state is None else state.to(torch.float32).contiguous()
+    s0 = None if state is None else _as(state, torch.float32)
     y = torch.empty(v.shape, dtype=odt, device=dev)
     s_out = torch.empty(N, Hv, Dv, Dk, dtype=torch.float32, device=dev)
     ckpt = None
     if save_ckpt:
-        ckpt = torch.empty(max(_lib.ckpt_bytes(desc) // 4, 1), dtype=torch.float32, device=dev)
-    ws = _workspace(desc, dev)
-    _lib.fwd(desc, _dev_ptr(q), _dev_ptr(k), _dev_ptr(v), _dev_ptr(g), _dev_ptr(beta), _dev_ptr(s0), _dev_ptr(y),
+        ckpt = torch.empty(plan.ckpt_floats, dtype=torch.float32, device=dev)
+    ws = _workspace(plan, dev)
+    _lib.fwd(plan, _dev_ptr(q), _dev_ptr(k), _dev_ptr(v), _dev_ptr(g), _dev_ptr(beta), _dev_ptr(s0), _dev_ptr(y),
              _dev_ptr(s_out), _dev_ptr(ckpt), _dev_ptr(ws), _stream(dev))
-    del keep
     return y, s_out, ckpt
 
 
@@ -99,24 +111,20 @@ def backward(q, k, v, g, beta, ckpt, dy, ds_out=None, *, log_decay=False, design
     dtype = _io_dtype(q, k, v, beta)
     q, k, v, g, beta = _prep(q, k, v, g, beta, dtype)
     odt = torch.float32 if out_f32 else dtype
-    dy = dy.to(odt).contiguous()
-    desc, keep = _desc(q, v, dtype, log_decay, design, cu_seqlens, out_f32)
-    why = _lib.validate(desc)
-    if why:
-        raise RuntimeError(why)
+    dy = _as(dy, odt)
+    plan = _plan(q, v, dtype, log_decay, design, cu_seqlens, out_f32)
     N = q.shape[0] if cu_seqlens is None else len(cu_seqlens) - 1
     dev = q.device
     Hv, Dv, Dk = v.shape[2], v.shape[3], q.shape[3]
-    dso = None if ds_out is None else ds_out.to(torch.float32).contiguous()
+    dso = None if ds_out is None else _as(ds_out, torch.float32)
     dq, dk = torch.empty(q.shape, dtype=odt, device=dev), torch.empty(k.shape, dtype=odt, device=dev)
     dv, dbeta = torch.empty(v.shape, dtype=odt, device=dev), torch.empty(beta.shape, dtype=odt, device=dev)
     dg = torch.empty_like(g)
     ds0 = torch.empty(N, Hv, Dv, Dk, dtype=torch.float32, device=dev) if want_ds0 else None
-    ws = _workspace(desc, dev)
-    _lib.bwd(desc, _dev_ptr(q), _dev_ptr(k), _dev_ptr(v), _dev_ptr(g), _dev_ptr(beta), _dev_ptr(ckpt), _dev_ptr(dy),
+    ws = _workspace(plan, dev)
+    _lib.bwd(plan, _dev_ptr(q), _dev_ptr(k), _dev_ptr(v), _dev_ptr(g), _dev_ptr(beta), _dev_ptr(ckpt), _dev_ptr(dy),
              _dev_ptr(dso), _dev_ptr(dq), _dev_ptr(dk), _dev_ptr(dv), _dev_ptr(dg), _dev_ptr(dbeta), _dev_ptr(ds0),
              _dev_ptr(ws), _stream(dev))
-    del keep
     return dq, dk, dv, dg, dbeta, ds0
 
 
@@ -129,26 +137,22 @@ def forward_prologue(q_raw, k_raw, v, a, b, a_log, dt_bias, state=None, *, cu_se
         if t.dtype != torch.bfloat16 or not t.is_cuda:
             raise RuntimeError("gated delta: the fused prologue takes bf16 device tensors")
     q_raw, k_raw, v, a, b = (t.contiguous() for t in (q_raw, k_raw, v, a, b))
-    a_log, dt_bias = a_log.float().contiguous(), dt_bias.float().contiguous()
-    desc, keep = _desc(q_raw, v, torch.bfloat16, True, _lib.CHUNKED, cu_seqlens, out_f32)
-    why = _lib.validate(desc)
-    if why:
-        raise RuntimeError(why)
+    a_log, dt_bias = _as(a_log, torch.float32), _as(dt_bias, torch.float32)
+    plan = _plan(q_raw, v, torch.bfloat16, True, _lib.CHUNKED, cu_seqlens, out_f32)
     N = q_raw.shape[0] if cu_seqlens is None else len(cu_seqlens) - 1
     dev = q_raw.device
     Hv, Dv, Dk = v.shape[2], v.shape[3], q_raw.shape[3]
-    s0 = None if state is None else state.to(torch.float32).contiguous()
+    s0 = None if state is None else _as(state, torch.float32)
     q, k = torch.empty_like(q_raw), torch.empty_like(k_raw)
     beta = torch.empty_like(b)
     log_decay = torch.empty(a.shape, dtype=torch.float32, device=dev)
     y = torch.empty(v.shape, dtype=torch.float32 if out_f32 else torch.bfloat16, device=dev)
     s_out = torch.empty(N, Hv, Dv, Dk, dtype=torch.float32, device=dev)
-    ckpt = torch.empty(max(_lib.ckpt_bytes(desc) // 4, 1), dtype=torch.float32, device=dev)
-    ws = _workspace(desc, dev)
-    _lib.fwd_prologue(desc, _dev_ptr(q_raw), _dev_ptr(k_raw), _dev_ptr(v), _dev_ptr(a), _dev_ptr(b), _dev_ptr(a_log),
+    ckpt = torch.empty(plan.ckpt_floats, dtype=torch.float32, device=dev)
+    ws = _workspace(plan, dev)
+    _lib.fwd_prologue(plan, _dev_ptr(q_raw), _dev_ptr(k_raw), _dev_ptr(v), _dev_ptr(a), _dev_ptr(b), _dev_ptr(a_log),
                       _dev_ptr(dt_bias), _dev_ptr(s0), _dev_ptr(q), _dev_ptr(k), _dev_ptr(beta), _dev_ptr(log_decay),
                       _dev_ptr(y), _dev_ptr(s_out), _dev_ptr(ckpt), _dev_ptr(ws), _stream(dev))
-    del keep
     return y, s_out, ckpt, q, k, beta, log_decay
 
 
@@ -163,27 +167,23 @@ def backward_prologue(q_raw, k_raw, a, b, a_log, dt_bias, q, k, v, beta, log_dec
         if t.dtype != torch.bfloat16 or not t.is_cuda:
             raise RuntimeError("gated delta: the fused prologue backward takes bf16 device tensors")
     q_raw, k_raw, a, b, q, k, v, beta, dy = (t.contiguous() for t in (q_raw, k_raw, a, b, q, k, v, beta, dy))
-    a_log, dt_bias = a_log.float().contiguous(), dt_bias.float().contiguous()
-    log_decay = log_decay.float().contiguous()
-    desc, keep = _desc(q_raw, v, torch.bfloat16, True, _lib.CHUNKED, cu_seqlens, False)
-    why = _lib.validate(desc)
-    if why:
-        raise RuntimeError(why)
+    a_log, dt_bias = _as(a_log, torch.float32), _as(dt_bias, torch.float32)
+    log_decay = _as(log_decay, torch.float32)
+    plan = _plan(q_raw, v, torch.bfloat16, True, _lib.CHUNKED, cu_seqlens, False)
     N = q_raw.shape[0] if cu_seqlens is None else len(cu_seqlens) - 1
     dev = q_raw.device
     Hv, Dv, Dk = v.shape[2], v.shape[3], q_raw.shape[3]
-    dso = None if ds_out is None else ds_out.to(torch.float32).contiguous()
+    dso = None if ds_out is None else _as(ds_out, torch.float32)
     dq_raw, dk_raw, dv = torch.empty_like(q_raw), torch.empty_like(k_raw), torch.empty_like(v)
     da, db = torch.empty_like(a), torch.empty_like(b)
     da_log, ddt_bias = torch.empty_like(a_log), torch.empty_like(dt_bias)
     ds0 = torch.empty(N, Hv, Dv, Dk, dtype=torch.float32, device=dev) if want_ds0 else None
-    ws = _workspace(desc, dev)
-    _lib.bwd_prologue(desc, _dev_ptr(q_raw), _dev_ptr(k_raw), _dev_ptr(a), _dev_ptr(b), _dev_ptr(a_log),
+    ws = _workspace(plan, dev)
+    _lib.bwd_prologue(plan, _dev_ptr(q_raw), _dev_ptr(k_raw), _dev_ptr(a), _dev_ptr(b), _dev_ptr(a_log),
                       _dev_ptr(dt_bias), _dev_ptr(q), _dev_ptr(k), _dev_ptr(v), _dev_ptr(beta), _dev_ptr(log_decay),
                       _dev_ptr(ckpt), _dev_ptr(dy), _dev_ptr(dso), _dev_ptr(dq_raw), _dev_ptr(dk_raw), _dev_ptr(dv),
                       _dev_ptr(da), _dev_ptr(db), _dev_ptr(da_log), _dev_ptr(ddt_bias), _dev_ptr(ds0), _dev_ptr(ws),
                       _stream(dev))
-    del keep
     return dq_raw, dk_raw, dv, da, db, da_log, ddt_bias, ds0
 
 
@@ -193,14 +193,13 @@ def forward_rows(q, k, v, g, beta, state=None, *, log_decay=False, cu_seqlens=No
     decoder rolls back to any row's state (src/exact.cpp:152-162). Runs the recurrent design."""
     dtype = _io_dtype(q, k, v, beta)
     q, k, v, g, beta = _prep(q, k, v, g, beta, dtype)
-    desc, keep = _desc(q, v, dtype, log_decay, _lib.RECURRENT, cu_seqlens, False)
+    plan = _plan(q, v, dtype, log_decay, _lib.RECURRENT, cu_seqlens, False)
     B, T, Hv, Dv = v.shape
     y = torch.empty(v.shape, dtype=dtype, device=v.device)
     rows = torch.empty((B, T, Hv, Dv, q.shape[-1]), dtype=torch.float32, device=v.device)
-    s0 = None if state is None else state.to(torch.float32).contiguous()
-    _lib.fwd_rows(desc, _dev_ptr(q), _dev_ptr(k), _dev_ptr(v), _dev_ptr(g), _dev_ptr(beta), _dev_ptr(s0),
+    s0 = None if state is None else _as(state, torch.float32)
+    _lib.fwd_rows(plan, _dev_ptr(q), _dev_ptr(k), _dev_ptr(v), _dev_ptr(g), _dev_ptr(beta), _dev_ptr(s0),
                   _dev_ptr(y), _dev_ptr(rows), _stream(q.device))
-    del keep
     if cu_seqlens is not None:
         rows = rows.view(B * T, Hv, Dv, q.shape[-1])
     return y, rows
@@ -216,6 +215,7 @@ class _GatedDelta(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, g, beta, ckpt)
         ctx.state_meta = (state is not None, None if state is None else state.dtype)
         ctx.opts = (log_decay, design)
+        ctx.set_materialize_grads(False)  # the final state mostly has no cotangent: none is better than zeros
         return y.to(q.dtype), s_out
 
     @staticmethod
@@ -224,8 +224,9 @@ class _GatedDelta(torch.autograd.Function):
         log_decay, design = ctx.opts
         if dy is None:
             dy = torch.zeros(v.shape, dtype=q.dtype, device=q.device)
-        dq, dk, dv, dg, dbeta, ds0 = backward(q, k, v, g, beta, ckpt, dy, dstate, log_decay=log_decay, design=design)
         has_state, sdt = ctx.state_meta
+        dq, dk, dv, dg, dbeta, ds0 = backward(q, k, v, g, beta, ckpt, dy, dstate, log_decay=log_decay, design=design,
+                                              want_ds0=has_state)
         return (dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), dg.to(g.dtype), dbeta.to(beta.dtype),
                 ds0.to(sdt) if has_state else None, None, None)
 
@@ -243,6 +244,7 @@ class _GatedDeltaPrologue(torch.autograd.Function):
         y, s_out, ckpt, q, k, beta, log_decay = forward_prologue(q_raw, k_raw, v, a, b, a_log, dt_bias, state)
         ctx.save_for_backward(q_raw, k_raw, a, b, a_log, dt_bias, q, k, v, beta, log_decay, ckpt)
         ctx.meta = (state is not None, None if state is None else state.dtype, a_log.dtype, dt_bias.dtype)
+        ctx.set_materialize_grads(False)
         return y, s_out
 
     @staticmethod

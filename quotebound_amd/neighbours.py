@@ -23,20 +23,28 @@ def _ptr(t):
 
 
 def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _act_dtype(*ts):
-    return torch.bfloat16 if all(t.dtype == torch.bfloat16 for t in ts) else torch.float32
+    return torch.bfloat16 if all([t.dtype == torch.bfloat16 for t in ts]) else torch.float32
 
 
-def _desc(B, T, Hk, Hv, Dk, Dv, dtype):
-    d, keep = _lib.make_desc(B, T, Hk, Hv, Dk, Dv, dtype=_lib.BF16 if dtype == torch.bfloat16 else _lib.F32)
-    return d, keep
+def _as(t, dtype):
+    """t in dtype, contiguous."""
+    return t if t.dtype == dtype and t.is_contiguous() else t.to(dtype).contiguous()
 
 
-def _ws(desc, device):
-    return torch.empty(max(_lib.neighbours_workspace_bytes(desc), 1), dtype=torch.uint8, device=device)
+def _plan(B, T, Hk, Hv, Dk, Dv, dtype):
+    def make():
+        desc, keep = _lib.make_desc(B, T, Hk, Hv, Dk, Dv, dtype=_lib.BF16 if dtype == torch.bfloat16 else _lib.F32)
+        return _lib.Plan(desc, keep, _lib.neighbours_workspace_bytes(desc))
+
+    return _lib.plan(("neighbours", B, T, Hk, Hv, Dk, Dv, dtype), make)
+
+
+def _ws(plan, device):
+    return torch.empty(plan.workspace, dtype=torch.uint8, device=device)
 
 
 def _check(*ts):
@@ -47,64 +55,60 @@ def _check(*ts):
 def prologue_forward(q_raw, k_raw, a, b, a_log, dt_bias):
     _check(q_raw, k_raw, a, b, a_log, dt_bias)
     dt = _act_dtype(q_raw, k_raw, a, b)
-    c = lambda t: t.to(dt).contiguous()  # noqa: E731
+    c = lambda t: _as(t, dt)  # noqa: E731
     q_raw, k_raw, a, b = c(q_raw), c(k_raw), c(a), c(b)
-    a_log, dt_bias = a_log.float().contiguous(), dt_bias.float().contiguous()
+    a_log, dt_bias = _as(a_log, torch.float32), _as(dt_bias, torch.float32)
     B, T, Hk, Dk = q_raw.shape
     Hv = a.shape[2]
-    desc, keep = _desc(B, T, Hk, Hv, Dk, Dk, dt)
+    plan = _plan(B, T, Hk, Hv, Dk, Dk, dt)
     q, k = torch.empty_like(q_raw), torch.empty_like(k_raw)
     beta = torch.empty_like(b)
     log_decay = torch.empty(a.shape, dtype=torch.float32, device=a.device)
-    _lib.prologue_fwd(desc, _ptr(q_raw), _ptr(k_raw), _ptr(a), _ptr(b), _ptr(a_log), _ptr(dt_bias), _ptr(q), _ptr(k),
+    _lib.prologue_fwd(plan, _ptr(q_raw), _ptr(k_raw), _ptr(a), _ptr(b), _ptr(a_log), _ptr(dt_bias), _ptr(q), _ptr(k),
                       _ptr(beta), _ptr(log_decay), _stream(a.device))
-    del keep
     return q, k, beta, log_decay
 
 
 def prologue_backward(q_raw, k_raw, a, b, a_log, dt_bias, dq, dk, dbeta, dlog_decay):
     """Returns (dq_raw, dk_raw, da, db, da_log, ddt_bias)."""
     dt = _act_dtype(q_raw, k_raw, a, b)
-    c = lambda t: t.to(dt).contiguous()  # noqa: E731
+    c = lambda t: _as(t, dt)  # noqa: E731
     q_raw, k_raw, a, b, dq, dk, dbeta = map(c, (q_raw, k_raw, a, b, dq, dk, dbeta))
-    a_log, dt_bias = a_log.float().contiguous(), dt_bias.float().contiguous()
-    dlog_decay = dlog_decay.float().contiguous()
+    a_log, dt_bias = _as(a_log, torch.float32), _as(dt_bias, torch.float32)
+    dlog_decay = _as(dlog_decay, torch.float32)
     B, T, Hk, Dk = q_raw.shape
     Hv = a.shape[2]
-    desc, keep = _desc(B, T, Hk, Hv, Dk, Dk, dt)
+    plan = _plan(B, T, Hk, Hv, Dk, Dk, dt)
     dq_raw, dk_raw, da, db = (torch.empty_like(t) for t in (q_raw, k_raw, a, b))
     da_log, ddt = torch.empty_like(a_log), torch.empty_like(dt_bias)
-    _lib.prologue_bwd(desc, _ptr(q_raw), _ptr(k_raw), _ptr(a), _ptr(b), _ptr(a_log), _ptr(dt_bias), _ptr(dq),
+    _lib.prologue_bwd(plan, _ptr(q_raw), _ptr(k_raw), _ptr(a), _ptr(b), _ptr(a_log), _ptr(dt_bias), _ptr(dq),
                       _ptr(dk), _ptr(dbeta), _ptr(dlog_decay), _ptr(dq_raw), _ptr(dk_raw), _ptr(da), _ptr(db),
-                      _ptr(da_log), _ptr(ddt), _ptr(_ws(desc, a.device)), _stream(a.device))
-    del keep
+                      _ptr(da_log), _ptr(ddt), _ptr(_ws(plan, a.device)), _stream(a.device))
     return dq_raw, dk_raw, da, db, da_log, ddt
 
 
 def epilogue_forward(y, z, norm_w, eps):
     _check(y, z, norm_w)
     dt = _act_dtype(y, z)
-    y, z = y.to(dt).contiguous(), z.to(dt).contiguous()
+    y, z = _as(y, dt), _as(z, dt)
     B, T, Hv, Dv = y.shape
-    desc, keep = _desc(B, T, Hv, Hv, Dv, Dv, dt)
+    plan = _plan(B, T, Hv, Hv, Dv, Dv, dt)
     o = torch.empty_like(y)
-    _lib.epilogue_fwd(desc, _ptr(y), _ptr(z), _ptr(norm_w.float().contiguous()), float(eps), _ptr(o),
+    _lib.epilogue_fwd(plan, _ptr(y), _ptr(z), _ptr(_as(norm_w, torch.float32)), float(eps), _ptr(o),
                       _stream(y.device))
-    del keep
     return o
 
 
 def epilogue_backward(y, z, norm_w, eps, dout):
     """Returns (dy, dz, dnorm_w)."""
     dt = _act_dtype(y, z)
-    y, z, dout = y.to(dt).contiguous(), z.to(dt).contiguous(), dout.to(dt).contiguous()
+    y, z, dout = _as(y, dt), _as(z, dt), _as(dout, dt)
     B, T, Hv, Dv = y.shape
-    desc, keep = _desc(B, T, Hv, Hv, Dv, Dv, dt)
-    w = norm_w.float().contiguous()
+    plan = _plan(B, T, Hv, Hv, Dv, Dv, dt)
+    w = _as(norm_w, torch.float32)
     dy, dz, dw = torch.empty_like(y), torch.empty_like(z), torch.empty_like(w)
-    _lib.epilogue_bwd(desc, _ptr(y), _ptr(z), _ptr(w), float(eps), _ptr(dout), _ptr(dy), _ptr(dz), _ptr(dw),
-                      _ptr(_ws(desc, y.device)), _stream(y.device))
-    del keep
+    _lib.epilogue_bwd(plan, _ptr(y), _ptr(z), _ptr(w), float(eps), _ptr(dout), _ptr(dy), _ptr(dz), _ptr(dw),
+                      _ptr(_ws(plan, y.device)), _stream(y.device))
     return dy, dz, dw
 
 
