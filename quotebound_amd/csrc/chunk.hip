@@ -12,7 +12,7 @@ ChunkLayout layout_of(const Problem& p) { return ChunkLayout{p.NC, p.Hv, p.Dv, p
 
 size_t extras_bytes(const Problem& p) { return layout_of(p).tiles_bytes(); }
 size_t dsend_bytes(const Problem& p) { return size_t(p.NC) * p.Hv * p.Dv * p.Dk * 4; }
-// The fused prologue backward's per-(chunk slot, value head) sums, after dSend.
+// The fused prologue backward's per-(chunk slot, value head) sums, or chunk_dgfix's list, after dSend.
 size_t gate_part_bytes(const Problem& p) { return (size_t(p.NC) * p.Hv * 2 * 4 + 255) & ~size_t(255); }
 
 // The current device's compute-unit count; 256 (MI355X) when it cannot be read, as with no device (host-only
@@ -139,6 +139,8 @@ hipError_t bwd_impl(const Problem& p, const PrologueGradIn* pro, const BwdPtrs& 
   a.dbeta = b.dbeta;
   a.ds0 = b.ds0;
   a.dsend = static_cast<float*>(ws);
+  // The list has the gate sums' place, which only the fused prologue uses (on log-decays).
+  if (!p.g_is_log) a.fix = reinterpret_cast<int*>(static_cast<unsigned char*>(ws) + dsend_bytes(p));
   if (split_grads(p))
     a.dqk_part = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + dsend_bytes(p) + gate_part_bytes(p));
   if (pro) {
@@ -159,8 +161,8 @@ hipError_t bwd_impl(const Problem& p, const PrologueGradIn* pro, const BwdPtrs& 
   // normalisation's backward.
   if (e == hipSuccess && a.dqk_part) e = launch_chunk_dqk_sum(a, p.out_bf16, s, pro != nullptr);
   if (e == hipSuccess && pro) e = launch_chunk_gate_sums(a, pro->da_log, pro->ddt_bias, s);
-  // With g given as the factor, dL/dg at tiny or zero factors comes from an exact replay (chunk_dgfix.hip); chunks
-  // without one return at once.
+  // With g given as the factor, dL/dg at tiny or zero factors comes from an exact replay (chunk_dgfix.hip) of the
+  // chunks that the gradient kernel listed.
   if (e == hipSuccess && !p.g_is_log) e = launch_chunk_dgfix(a, p.out_bf16, s);
   tr.mark();
   return e;

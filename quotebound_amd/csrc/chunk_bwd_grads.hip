@@ -607,12 +607,17 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
           pa = sum16(pa), pd = sum16(pd);
           pa = swap32_sum(swap16_sum(pa)), pd = swap32_sum(swap16_sum(pd));
           if (t == 0) a.pro.part[(slot * a.Hv + hv) * 2] = pa, a.pro.part[(slot * a.Hv + hv) * 2 + 1] = pd;
-        } else if (t < L) {
+        } else {
           const int64_t g0 = tok * a.Hv + hv;
           const uint32_t gi = uint32_t(t * a.Hv);
-          a.dg[g0 + gi] = a.g_is_log ? v : v / a.g[g0 + gi];
-          const float dbT = bpos[0][t] + bpos[1][t];
-          IO<OutT>::st(static_cast<OutT*>(a.dbeta) + g0, gi, dbT + dbA);
+          const float gx = !a.g_is_log && t < L ? a.g[g0 + gi] : 1.f;
+          if (t < L) {
+            a.dg[g0 + gi] = v / gx;
+            const float dbT = bpos[0][t] + bpos[1][t];
+            IO<OutT>::st(static_cast<OutT*>(a.dbeta) + g0, gi, dbT + dbA);
+          }
+          if (a.fix && __ballot(!(gx >= kTinyFactor)) != 0 && tid == 0)
+            a.fix[1 + atomicAdd(a.fix, 1)] = int(slot) * a.Hv + hv;
         }
       }
     }

@@ -52,6 +52,7 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_state_kernel(ChunkArgs a) 
   __shared__ __align__(16) float Xs[kRows * kLX];
   __shared__ float Gs[2][3 * kC];  // exp G, D, beta, by chunk parity
 
+  if (a.fix && blockIdx.x == 0 && threadIdx.x == 0) *a.fix = 0;
   const int total = a.nblk * a.Hv * a.N;
   const StateItem item = state_item(a.tab, blockIdx.x, a.nblk, a.Hv, a.Hk, total);
   const int blk = item.blk, hv = item.hv, n = item.n;

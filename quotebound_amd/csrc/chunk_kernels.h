@@ -5,6 +5,8 @@
 
 namespace qbgdn {
 
+constexpr float kTinyFactor = 0x1p-10f;  // decay factors below this take chunk_dgfix's dL/dg
+
 struct ChunkArgs {
   const bf16_t* q;
   const bf16_t* k;
@@ -25,6 +27,10 @@ struct ChunkArgs {
   void* dbeta;
   float* ds0;
   float* dsend;  // workspace: cotangent of each chunk's end state
+  // Workspace, with g given as the factor: how many (chunk slot, value head) pairs hold a factor below kTinyFactor, then
+  // the pairs (slot * Hv + head), in no order. Cleared by the backward state pass, listed by the gradient kernel, taken
+  // up by chunk_dgfix.
+  int* fix;
   float* dqk_part;  // workspace, short sequences: per (chunk slot, value head) dq and dk [64][128] float32, or null
   ChunkLayout lay;
   int Hk, Hv, Dv, g_is_log;
