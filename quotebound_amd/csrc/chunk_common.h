@@ -67,6 +67,28 @@ __device__ __forceinline__ bf16x8 tri_tr8(const __bf16* M, int r0, int J, int la
   return in ? v : z;
 }
 
+// The inverse of I + A for strictly lower triangular 16 x 16 matrices A, one per row of 16 lanes, by substitution: lane
+// jl brings its column of A, a[il] = A[il][jl], and gets column jl of the inverse. A row's entries reach the other
+// lanes by DPP (row_newbcast), so a step is vector instructions alone; read from LDS, each of the 120 entries is a
+// round trip's share of one wave's time while the block waits.
+template <int IL, int KL>
+__device__ __forceinline__ void lower_inverse16_row(float& v, const float (&a)[16], const float (&x)[16]) {
+  if constexpr (KL < IL) {
+    const float b = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a[IL]), 0x150 + KL, 0xf, 0xf, true));
+    v -= b * x[KL];  // x[KL] = 0 for KL < jl
+    lower_inverse16_row<IL, KL + 1>(v, a, x);
+  }
+}
+template <int IL = 0>
+__device__ __forceinline__ void lower_inverse16(const float (&a)[16], float (&x)[16], int jl) {
+  if constexpr (IL < 16) {
+    float v = IL == jl ? 1.f : 0.f;
+    lower_inverse16_row<IL, 0>(v, a, x);
+    x[IL] = IL >= jl ? v : 0.f;
+    lower_inverse16<IL + 1>(a, x, jl);
+  }
+}
+
 struct ChunkLayout {
   int64_t NC;
   int Hv, Dv, Dk;

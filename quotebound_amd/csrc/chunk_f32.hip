@@ -208,19 +208,16 @@ __global__ __launch_bounds__(256, 4) void f32_prep_kernel(F32Args a, int hpb) {
         neg = !a.g_is_log && gx < 0.f;
       }
       const uint64_t nm = __ballot(neg);
-#pragma unroll
-      for (int off = 1; off < kC; off <<= 1) {
-        const double u = __shfl_up(G, off);
-        if (tid >= off) G += u;
-      }
-      const double Glast = __shfl(G, kC - 1);
-      const float sg = __popcll(nm & ((uint64_t(2) << tid) - 1)) & 1 ? -1.f : 1.f, sl = __popcll(nm) & 1 ? -1.f : 1.f;
-      Gd[tid] = G, Bs[tid] = bx, Sg[tid] = sg;
-      tile->gam[tid] = sg * expf(float(G));
-      tile->dec[tid] = sg * sl * expf(float(Glast - G));
-      tile->beta[tid] = bx;
+      Gd[tid] = wave_prefix_sum(G), Bs[tid] = bx;
+      Sg[tid] = __popcll(nm & ((uint64_t(2) << tid) - 1)) & 1 ? -1.f : 1.f;
     }
     __syncthreads();
+    if (w == 3) {  // the tile's vectors: a wave with two blocks where two others have three
+      const double G = Gd[lane], Glast = Gd[kC - 1];
+      tile->gam[lane] = Sg[lane] * expf(float(G));
+      tile->dec[lane] = Sg[lane] * Sg[kC - 1] * expf(float(Glast - G));
+      tile->beta[lane] = Bs[lane];
+    }
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       const int b = w + 4 * u, I = (b >= 1) + (b >= 3) + (b >= 6), J = b - I * (I + 1) / 2;
@@ -245,14 +242,10 @@ __global__ __launch_bounds__(256, 4) void f32_prep_kernel(F32Args a, int hpb) {
     // T_IJ = -T_II sum_{J <= K < I} A_IK T_KJ, one wave per block.
     if (tid < kC) {
       const int jl = tid & 15, b0 = tid & ~15;
-      float x[16];
+      float x[16], col[16];
 #pragma unroll
-      for (int il = 0; il < 16; ++il) {
-        float v = il == jl ? 1.f : 0.f;
-#pragma unroll
-        for (int kl = 0; kl < il; ++kl) v = kl >= jl ? v - Am[tri_pad(b0 + il, b0 + kl)] * x[kl] : v;
-        x[il] = il >= jl ? v : 0.f;
-      }
+      for (int il = 0; il < 16; ++il) col[il] = Am[tri_pad(b0 + il, b0 + jl)];
+      lower_inverse16(col, x, jl);
 #pragma unroll
       for (int il = 0; il < 16; ++il) Tm[tri_pad(b0 + il, b0 + jl)] = x[il];
     }

@@ -173,28 +173,25 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(ChunkArgs a, int h
     // The first pass: every wave is done with the k and q rows. Later ones: done with the previous head's G, beta,
     // A, T and P.
     __syncthreads();
-    // One wave: G = the inclusive prefix sum of the log-decays, accumulated in fp64 by a shuffle scan (so G_i - G_j
+    // One wave: G = the inclusive prefix sum of the log-decays, accumulated in fp64 by a DPP scan (so G_i - G_j
     // keeps its bits when |G| is large). Then the next value head's scalars are read, to arrive during this head.
     if (tid < kC) {
       const int t = tid;
       // The log-decay floored at -150: a factor of 0 (or a log-decay of -inf) would make G_i - G_j NaN on every pair
       // across it; at -150 each exp(.) across it is 0 in float32, as the factor 0 makes it.
       double G = uint32_t(t) < L ? fmax(kFused || a.g_is_log ? double(gx) : double(logf(gx)), kLogFloor) : 0.0;
-#pragma unroll
-      for (int off = 1; off < kC; off <<= 1) {
-        const double u = __shfl_up(G, off);
-        if (t >= off) G += u;
-      }
-      const double Glast = __shfl(G, kC - 1);
-      Gd[t] = G;
+      Gd[t] = wave_prefix_sum(G);
       Bs[t] = uint32_t(t) < L ? bx : 0.f;
-      tile->beta[t] = Bs[t];
-      tile->gam[t] = expf(float(G));
-      tile->dec[t] = expf(float(Glast - G));
-      tile->G[t] = float(G);
       if (vh + 1 < hpb) load_scalars(hv + 1, gx, bx);
     }
     __syncthreads();
+    if (w == 3) {  // the tile's vectors: a wave with two blocks where two others have three
+      const double G = Gd[lane], Glast = Gd[kC - 1];
+      tile->beta[lane] = Bs[lane];
+      tile->gam[lane] = expf(float(G));
+      tile->dec[lane] = expf(float(Glast - G));
+      tile->G[lane] = float(G);
+    }
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       const int b = w + 4 * u;
@@ -227,14 +224,10 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(ChunkArgs a, int h
     // Diagonal blocks: thread -> column j of block bd; the column lives in registers through the substitution.
     if (tid < kC) {
       const int bd = tid >> 4, jl = tid & 15, b0 = 16 * bd;
-      float x[16];
+      float x[16], col[16];
 #pragma unroll
-      for (int il = 0; il < 16; ++il) {
-        float v = il == jl ? 1.f : 0.f;
-#pragma unroll
-        for (int kl = 0; kl < il; ++kl) v -= Am[tri_pad(b0 + il, b0 + kl)] * x[kl];  // x[kl] = 0 for kl < jl
-        x[il] = il >= jl ? v : 0.f;
-      }
+      for (int il = 0; il < 16; ++il) col[il] = Am[tri_pad(b0 + il, b0 + jl)];
+      lower_inverse16(col, x, jl);
 #pragma unroll
       for (int il = 0; il < 16; ++il) Tm[tri_pad(b0 + il, b0 + jl)] = x[il];
     }

@@ -4,8 +4,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
-
 namespace qbgdn {
 
 constexpr int kChunk = 64;     // checkpoint stride, the reference's kChunk (src/delta_grad.cpp:11)
@@ -112,9 +110,10 @@ struct BufIO<bf16_t> {
 
 // ---- lane reductions ------------------------------------------------------------------------------------------
 // DPP controls (gfx9 encoding): quad_perm, row_mirror, row_half_mirror.
-template <int CTRL>
+// (ROWS: the rows of 16 lanes that take part; the others, and lanes without a source, get 0.)
+template <int CTRL, int ROWS = 0xf>
 __device__ __forceinline__ float dpp_mov(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROWS, 0xf, false));
 }
 
 // Sum over each 16-lane row of the wave; every lane of the row gets the same bits (each stage pairs lanes
@@ -152,21 +151,26 @@ __device__ __forceinline__ void sum32_pair(float& a, float& b) {
   b = __uint_as_float(t[1]);
 }
 
-// The inclusive prefix sum over the wave's 64 lanes: within each row of 16 lanes by row_shr 1, 2, 4, 8 (lanes without
-// a source add zero), then row 0's total into row 1 and row 2's into row 3 (row_bcast 15), then the first two rows'
-// into the last two (row_bcast 31). VALU only, where six __shfl steps are LDS round trips.
-__device__ __forceinline__ float wave_prefix_sum(float x) {
-  const auto add = [&x](auto ctrl, auto rows) {
-    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, decltype(rows)::value,
-                                                    0xf, false));
-  };
-  using std::integral_constant;
-  add(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});
-  add(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
-  add(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
-  add(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
-  add(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});
-  add(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
+// The same of 64 bits.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp_mov(double x) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(b)), CTRL, ROWS, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)), CTRL, ROWS, 0xf, false);
+  return __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+}
+
+// The inclusive prefix sum over the wave's 64 lanes (float or double): within each row of 16 lanes by row_shr 1, 2, 4,
+// 8 (lanes without a source add zero), then row 0's total into row 1 and row 2's into row 3 (row_bcast 15), then the
+// first two rows' into the last two (row_bcast 31). VALU only, where six __shfl steps are LDS round trips.
+template <typename T>
+__device__ __forceinline__ T wave_prefix_sum(T x) {
+  x += dpp_mov<0x111>(x);
+  x += dpp_mov<0x112>(x);
+  x += dpp_mov<0x114>(x);
+  x += dpp_mov<0x118>(x);
+  x += dpp_mov<0x142, 0xa>(x);
+  x += dpp_mov<0x143, 0xc>(x);
   return x;
 }
 
