@@ -743,7 +743,9 @@ __global__ __launch_bounds__(512) void f32_bwd_grads_kernel(F32Args a) {
   __shared__ float vpos[2][kC], hpos[2][kC], bpos[kC], red[8];
   const int grp = a.Hv / a.Hk, total = int(a.NC) * a.Hk;
   const int tid = threadIdx.x;
-  const int pw = __builtin_amdgcn_readfirstlane((tid >> 6) & 3), hw = __builtin_amdgcn_readfirstlane(tid >> 8);
+  // The two waves of a SIMD hold position tiles p and 3 - p: the triangular products, which grow with p, even out.
+  const int hw = __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int pw = __builtin_amdgcn_readfirstlane(((tid >> 6) ^ (3 * (tid >> 8))) & 3);
   const int sk = a.Hk * Dk, sv = a.Hv * a.Dv, nb = a.Dv / kBlk;
   // The lane's places, re-formed where they are used from an opaque copy of the thread index, so that their address
   // expressions are not held (spilled) across the loops.
@@ -865,7 +867,7 @@ __global__ __launch_bounds__(512) void f32_bwd_grads_kernel(F32Args a) {
           put_block(sm + ((b + 1) & 1) * kBuf);
           load_next(b + 2);
         }
-#pragma unroll
+#pragma unroll 1
         for (int s = 0; s < 2; ++s) {
           const int at = psw(ip, 16 * s + 4 * g);
           const f32x4 ya = ld4(buf + oY + at), wa = ld4(buf + oW + at), ea = ld4(buf + oE + at);
