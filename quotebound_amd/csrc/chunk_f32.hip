@@ -24,8 +24,8 @@
 // operands follow the same order.
 //
 // Bound by the matrix pipes' float32 rate (256 operations a cycle and CU) and the latency of the chain of products in
-// the state passes: about half of that rate each. At B = 1, T = 4096, 16 key and 32 value heads of 128: prep 45 us,
-// forward 217, prep again 44, backward state pass 215, gradients 307, where the step-by-step kernels took 819 us
+// the state passes: about half of that rate each. At B = 1, T = 4096, 16 key and 32 value heads of 128: prep 38 us,
+// forward 218, prep again 39, backward state pass 214, gradients 299, where the step-by-step kernels took 819 us
 // forward and 1,877 + 202 backward.
 //
 // Every sum is taken 16 terms at a time from zero (four instructions) and the partial sums added up: a chain of 128
@@ -377,7 +377,7 @@ __device__ __forceinline__ f32x4 tri_cols(const float* m, const float* A, int wp
 // Waves 0-3 carry the state (wave w: positions 16w .., then state columns 32w ..), waves 4-7 form y, waves 8-11 load
 // the next chunk's inputs into registers a chunk ahead and stage them in LDS where their last readers are done. Three
 // barriers per chunk: S in LDS | K S^T, R | e, Delta | the update of S; y's S Q^T runs beside the first two and its P
-// Delta beside the third. A block issues 464 matrix instructions per chunk, 3,712 cycles on its four pipes.
+// Delta beside the third (S Q^T whole beside the second: 247 -> 239 us at 4,096 steps, 63.8 -> 64.6 at 777). A block issues 464 matrix instructions per chunk, 3,712 cycles on its four pipes.
 __global__ __launch_bounds__(768) void f32_fwd_kernel(F32Args a) {
   __shared__ __align__(16) float Sm[2][kR * Dk], Kb[2][kC * Dk], Qb[kC * Dk], Tb[kTri], Pb[kTri];
   __shared__ __align__(16) float Wr[kC * kLW], Wd[kC * kLW], We[kC * kLW], Vs[kC * kR], Gs[2][256];

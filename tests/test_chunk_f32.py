@@ -119,3 +119,61 @@ def test_not_finite(torch_dev, oracle, where):
         assert not np.isnan(got["y"]).any() and not np.isnan(got["dq"][0, 101:]).any()
         assert np.isnan(got["ds0"][0, 2, 17]).all() and np.isnan(got["ds0"]).sum() == 128
         assert normwise(got["dv"][~bad], clean["dv"][~bad]) <= TOL
+
+
+def _device(torch, inp):
+    return {n: torch.tensor(x).cuda() for n, x in inp.items()}
+
+
+def test_element_alignment(torch_dev):
+    """v, g, beta, dy and the states need only their elements' alignment: one float past a 16-byte boundary gives the
+    same bits."""
+    torch = torch_dev
+    from quotebound_amd import gdn
+
+    d = _device(torch, _float32(small_case(1, 200, 2, 4, 128, 64, seed=10)))
+
+    def off(t):
+        x = torch.empty(t.numel() + 1, device="cuda")[1:].view(t.shape)
+        return x.copy_(t)
+
+    def both(d):
+        five = (d["q"], d["k"], d["v"], d["g"], d["beta"])
+        y, s_out, ckpt = gdn.forward(*five, d["s0"], log_decay=True)
+        return [y, s_out, *gdn.backward(*five, ckpt, d["dy"], d["ds_out"], log_decay=True)]
+
+    moved = {n: t if n in ("q", "k") else off(t) for n, t in d.items()}
+    assert all(moved[n].data_ptr() % 16 == 4 for n in ("v", "g", "beta", "dy", "s0", "ds_out"))
+    assert all(torch.equal(x, y) for x, y in zip(both(d), both(moved)))
+
+
+def test_in_a_graph(torch_dev):
+    """Captured in a HIP graph: replays on new inputs give the eager call's bits, with eager work between them, and a
+    value that is not finite raises the flag in the replay that has it and in no other."""
+    torch = torch_dev
+    from quotebound_amd import gdn
+
+    def call(d):
+        five = (d["q"], d["k"], d["v"], d["g"], d["beta"])
+        y, s_out, ckpt = gdn.forward(*five, d["s0"], log_decay=True)
+        return [y, s_out, *gdn.backward(*five, ckpt, d["dy"], d["ds_out"], log_decay=True)]
+
+    cases = [_device(torch, _float32(small_case(1, 200, 2, 4, 128, 64, seed=s))) for s in (20, 21, 22)]
+    cases[1]["v"][0, 150, 1, 3] = float("nan")
+    static = {n: t.clone() for n, t in cases[0].items()}
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(static)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call(static)
+    for c in (cases[0], cases[1], cases[2], cases[0]):
+        want = call(c)
+        for n, t in static.items():
+            t.copy_(c[n])
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, y in zip(out, want):
+            assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.nan_to_num(), y.nan_to_num())
