@@ -1059,6 +1059,8 @@ void launch_prep(const F32Args& a, int cus, hipStream_t s) {
 
 bool chunk_f32_takes(const Problem& p, int steps, size_t ws_bytes) {
   if (p.in_bf16 || p.Dk != Dk || p.Dv % kBlk) return false;
+  // A chunk's rows of k and of v are addressed by 32-bit byte offsets.
+  if (int64_t(p.Hk) * Dk * kC * 4 >= (int64_t(1) << 31) || int64_t(p.Hv) * p.Dv * kC * 4 >= (int64_t(1) << 31)) return false;
   int longest = p.T;
   if (p.tab.n > 0) {
     longest = 0;
