@@ -139,8 +139,9 @@ hipError_t bwd_impl(const Problem& p, const PrologueGradIn* pro, const BwdPtrs& 
   a.dbeta = b.dbeta;
   a.ds0 = b.ds0;
   a.dsend = static_cast<float*>(ws);
-  // The list has the gate sums' place, which only the fused prologue uses (on log-decays).
-  if (!p.g_is_log) a.fix = reinterpret_cast<int*>(static_cast<unsigned char*>(ws) + dsend_bytes(p));
+  // The list has the gate sums' place, which only the fused prologue uses (on log-decays). With no chunk slots the
+  // workspace has no bytes, and the state pass, which clears the list's count, must be given no list.
+  if (!p.g_is_log && p.NC > 0) a.fix = reinterpret_cast<int*>(static_cast<unsigned char*>(ws) + dsend_bytes(p));
   if (split_grads(p))
     a.dqk_part = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + dsend_bytes(p) + gate_part_bytes(p));
   if (pro) {

@@ -1,5 +1,6 @@
 """dL/dg at tiny decay factors where more (chunk, value head) pairs hold one than the device has CUs, so that the
-blocks of the exact replay each take several of the listed pairs, and where none does, so that the list is empty.
+blocks of the exact replay each take several of the listed pairs, and where none does, so that the list is empty; and
+with no tokens, where the workspace that holds the list has no bytes.
 Against the oracle, within the 2e-3 of each output's largest value that the other tests of bf16 inputs allow (one
 rounding of the inputs, hi/lo products)."""
 import numpy as np
@@ -43,3 +44,26 @@ def test_listed_pairs(oracle, every):
     for name, x, y, e in zip(("dq", "dk", "dv", "dg", "dbeta", "ds0"), got, again, exp):
         assert torch.equal(x, y), name
         assert normwise(x.cpu().numpy(), e) <= 2e-3, (name, normwise(x.cpu().numpy(), e))
+
+
+@pytest.mark.parametrize("cu", [None, [0, 0, 0, 0]], ids=["batch", "packed"])
+@pytest.mark.parametrize("design", [_lib.CHUNKED, _lib.RECURRENT], ids=["chunked", "recurrent"])
+def test_no_tokens_leave_the_workspace_alone(design, cu):
+    """T = 0 asks for 0 bytes of workspace: whatever the pointer points at stays as it was, forward and backward, and
+    the final state is S0 and dS0 its cotangent."""
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    B, N, Hk, Hv, D = (3 if cu is None else 1), 3, 2, 4, 128
+    desc, keep = _lib.make_desc(B, 0, Hk, Hv, D, D, dtype=_lib.BF16, g_is_log=False, design=design, cu_seqlens=cu)
+    assert _lib.validate(desc) is None and _lib.workspace_bytes(desc) == 0
+    s0, ds_out = torch.randn(N, Hv, D, D, device="cuda"), torch.randn(N, Hv, D, D, device="cuda")
+    s_out, ds0 = torch.empty_like(s0), torch.empty_like(s0)
+    other = torch.full((256,), 0x5A, dtype=torch.uint8, device="cuda")
+    p, none, stream = (lambda t: t.data_ptr()), [None] * 5, torch.cuda.current_stream().cuda_stream
+    _lib.fwd(desc, *none, p(s0), None, p(s_out), None, p(other), stream)
+    _lib.bwd(desc, *none, None, None, p(ds_out), *none, p(ds0), p(other), stream)
+    torch.cuda.synchronize()
+    assert torch.equal(s_out, s0) and torch.equal(ds0, ds_out)
+    assert bool((other == 0x5A).all())
