@@ -299,7 +299,7 @@ namespace {
 // the library runs on holds until the process ends. In host code the name `scratch` is not a device address: the
 // array's address on a device comes from hipGetSymbolAddress, looked up once per device (the first call on it,
 // with that device current) and kept in scratch_ptr.
-static __device__ __align__(256) unsigned char scratch[QB_GDN_STATIC_SCRATCH_BYTES + 256];  // and the flag word
+static __device__ __align__(256) unsigned char scratch[QB_GDN_STATIC_SCRATCH_BYTES];
 constexpr int kMaxDevices = 64;
 std::atomic<void*> scratch_ptr[kMaxDevices];
 std::mutex scratch_mu;
@@ -334,8 +334,7 @@ int bwd_impl(const qb_gdn_desc* desc, const void* q, const void* k, const void* 
     const size_t el = p.in_bf16 ? 2 : 4, eo = p.out_bf16 ? 2 : 4;
     const bool any = p.BT > 0;
     const size_t need = why.empty() ? ws_bytes(desc, p) : 0;
-    const size_t flag = why.empty() && desc->design == QB_GDN_RECURRENT ? qbgdn::rec_flag_bytes(p) : 0;
-    if (why.empty() && use_static && need - flag > QB_GDN_STATIC_SCRATCH_BYTES)
+    if (why.empty() && use_static && need > QB_GDN_STATIC_SCRATCH_BYTES)
       why = "gated delta: the backward without allocation needs " + std::to_string(need) +
             " bytes of scratch, more than its static " + std::to_string(size_t(QB_GDN_STATIC_SCRATCH_BYTES)) + " " +
             shape_of(*desc);

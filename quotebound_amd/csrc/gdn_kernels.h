@@ -67,7 +67,6 @@ struct Tracer {
 const char* rec_supports(const Problem& p);  // null when supported, else why not
 size_t rec_ckpt_bytes(const Problem& p);
 size_t rec_workspace_bytes(const Problem& p);
-size_t rec_flag_bytes(const Problem& p);  // of those, the ones after the partials
 extern const char* const kRecFwdLaunches;  // comma-separated kernel names, in launch order
 extern const char* const kRecBwdLaunches;
 hipError_t rec_fwd(const Problem& p, const FwdPtrs& a, void* ws, hipStream_t s, Tracer& tr);
@@ -83,17 +82,6 @@ hipError_t rec_wide_fwd(const Problem& p, const FwdPtrs& ptrs, hipStream_t s);
 template <typename InT, typename OutT>
 hipError_t rec_wide_bwd(const Problem& p, const BwdPtrs& ptrs, float* dq_part, float* dk_part, float* dg_part,
                         float* db_part, float* scratch, int nblk, hipStream_t s);
-
-// Design 1 on float32 inputs at Dk = 128 over long sequences (chunk_f32.hip), with design 1's residuals and results.
-// They take calls whose longest sequence has at least this many steps. Both ways measured at 16 key and 32 value heads
-// (2 and 4 heads cross at the same lengths), forward then backward, us: 30 and 79 step by step against 34 and 106 at
-// 128 steps, 54 and 136 against 40 and 113 at 256.
-constexpr int kChunkF32FwdSteps = 160, kChunkF32BwdSteps = 192;
-// Whether they take the call within ws_bytes of workspace. They use the word at ws + flag_at besides, and *redo points
-// at it: not zero after them where the recurrent kernels must do the work again.
-bool chunk_f32_takes(const Problem& p, int steps, size_t ws_bytes);
-hipError_t chunk_f32_fwd(const Problem& p, const FwdPtrs& a, void* ws, size_t flag_at, const int** redo, hipStream_t s);
-hipError_t chunk_f32_bwd(const Problem& p, const BwdPtrs& a, void* ws, size_t flag_at, const int** redo, hipStream_t s);
 
 // Design 2: chunkwise WY/UT form on MFMA.
 const char* chunk_supports(const Problem& p);

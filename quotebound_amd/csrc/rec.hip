@@ -11,8 +11,6 @@
 // products taken on the previous state, so one reduction latency per step sits on the dependency chain:
 //   a = S_prev k, b = S_prev q;  u = g a;  delta = beta (v - u);  y = g b + delta (k.q);  S = g S_prev + delta k^T
 // The chunk-start states (the reference's ckpt, src/delta_grad.cpp:172-181) are written as the forward passes them.
-// Long sequences of float32 inputs at Dk = 128 run chunkwise on the matrix pipes instead (chunk_f32.hip), with these
-// kernels behind them for values that are not finite.
 // A call of one token per sequence that keeps neither checkpoints nor per-token states (decode) runs the same step
 // in rec_step_kernel, which reads its inputs straight into registers instead of staging a chunk.
 //
@@ -69,7 +67,6 @@ __device__ __forceinline__ int col_of(int cl, int i) {
 
 struct RecFwdArgs {
   FwdPtrs p;
-  const int* only;  // when set, the kernel runs only if the word it points at is not zero (chunk_f32.hip's flag)
   float* e_res;  // v - u per token and state row [tokens, Hv, Dv], after the states in ckpt (null without ckpt)
   int Hk, Hv, Dv, g_is_log, nblk, total;
   SeqTable tab;
@@ -77,7 +74,6 @@ struct RecFwdArgs {
 
 struct RecBwdArgs {
   BwdPtrs p;
-  const int* only;  // as in RecFwdArgs
   const float* e_res;  // the forward's v - u per token and state row
   int Hk, Hv, Dv, g_is_log, nblk, total;
   float* dq_part;  // [BT, Hv, nblk, Dk]
@@ -168,7 +164,6 @@ __global__ __launch_bounds__((Layout<NPT, LPR>::kThreads)) void rec_fwd_kernel(R
   auto Ks = reinterpret_cast<float (*)[Dk]>(lds + oK);
   auto Qs = reinterpret_cast<float (*)[Dk]>(lds + oQ);
 
-  if (a.only && *a.only == 0) return;
   const Item it = item_of(a.tab, a.nblk, a.Hv, a.Hk, a.total);
   const int tid = threadIdx.x, lane = tid & 63;
   const int cl = lane % LPR, rl = (tid >> 6) * Lay::kRowsPerWave + lane / LPR;
@@ -400,7 +395,6 @@ __global__ __launch_bounds__((Layout<NPT, LPR>::kThreads)) void rec_bwd_kernel(R
   auto Ks = reinterpret_cast<float (*)[Dk]>(lds + oK);
   auto Qs = reinterpret_cast<float (*)[Dk]>(lds + oQ);
 
-  if (a.only && *a.only == 0) return;
   const Item it = item_of(a.tab, a.nblk, a.Hv, a.Hk, a.total);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cl = lane % LPR, rl = wave * Lay::kRowsPerWave + lane / LPR;
@@ -588,9 +582,7 @@ template <typename OutT>
 __global__ __launch_bounds__(256) void rec_reduce_kernel(const float* dq_part, const float* dk_part,
                                                          const float* dg_part, const float* db_part, const float* g,
                                                          OutT* dq, OutT* dk, float* dg, OutT* dbeta, int Hk, int Hv,
-                                                         int Dk, int nblk, int g_is_log, int64_t items,
-                                                         const int* only) {
-  if (only && *only == 0) return;
+                                                         int Dk, int nblk, int g_is_log, int64_t items) {
   // Eight (token, key head) items per block, 32 lanes each, four columns per lane: an item's partials are
   // grp * nblk contiguous rows of Dk floats, read as 16-byte units and summed in row order (value head, then row
   // block), the fixed order of the reference (src/delta_grad.cpp:194-198 over row blocks).
@@ -653,17 +645,10 @@ int row_blocks(const Problem& p) {
   return (p.Dv + rows - 1) / rows;
 }
 
-// The recurrent kernels' partials of a backward; the float32 chunk kernels, where they run, need no more.
-size_t parts_bytes(const Problem& p) {
-  const size_t nblk = row_blocks(p);
-  return (2 * size_t(p.BT) * p.Hv * nblk * p.Dk + 2 * size_t(p.BT) * p.Hv * nblk) * sizeof(float);
-}
-
 template <typename InT, typename OutT>
-hipError_t launch_fwd(const Problem& p, const FwdPtrs& ptrs, void* ws, hipStream_t s, Tracer& tr) {
+hipError_t launch_fwd(const Problem& p, const FwdPtrs& ptrs, hipStream_t s, Tracer& tr) {
   RecFwdArgs a;
   a.p = ptrs;
-  a.only = nullptr;
   a.e_res = ptrs.ckpt ? ptrs.ckpt + int64_t(p.NC) * p.Hv * p.Dv * p.Dk : nullptr;
   a.Hk = p.Hk, a.Hv = p.Hv, a.Dv = p.Dv, a.g_is_log = p.g_is_log;
   a.nblk = row_blocks(p);
@@ -677,10 +662,6 @@ hipError_t launch_fwd(const Problem& p, const FwdPtrs& ptrs, void* ws, hipStream
     return e;
   }
   const bool rows = ptrs.rows != nullptr;
-  if (!rows && chunk_f32_takes(p, kChunkF32FwdSteps, parts_bytes(p))) {
-    const hipError_t e = chunk_f32_fwd(p, ptrs, ws, parts_bytes(p), &a.only, s);
-    if (e != hipSuccess) return e;
-  }
   // One token or none per sequence (batch mode with T = 1; packed, where every sequence that is not empty has one
   // chunk slot per token), with nothing to keep but y and the final state: the one-token step.
   const bool one = (p.tab.n == 0 ? p.T <= 1 : p.NC == p.BT) && !ptrs.ckpt && !rows;
@@ -715,7 +696,6 @@ template <typename InT, typename OutT>
 hipError_t launch_bwd(const Problem& p, const BwdPtrs& ptrs, void* ws, hipStream_t s, Tracer& tr) {
   RecBwdArgs a;
   a.p = ptrs;
-  a.only = nullptr;
   a.e_res = ptrs.ckpt + int64_t(p.NC) * p.Hv * p.Dv * p.Dk;
   a.Hk = p.Hk, a.Hv = p.Hv, a.Dv = p.Dv, a.g_is_log = p.g_is_log;
   a.nblk = row_blocks(p);
@@ -729,12 +709,6 @@ hipError_t launch_bwd(const Problem& p, const BwdPtrs& ptrs, void* ws, hipStream
   if (p.Dk > 256) {  // one wave per row (rec_wide.hip)
     e = rec_wide_bwd<InT, OutT>(p, ptrs, w.dq_part, w.dk_part, w.dg_part, w.db_part, w.scratch, a.nblk, s);
   } else {
-    // With g given as the factor, dL/dg is d/d(log-decay) / g, whose rounding a small g magnifies: those calls keep
-    // the step-by-step backward, which forms dL/dg itself.
-    if (p.g_is_log && chunk_f32_takes(p, kChunkF32BwdSteps, parts_bytes(p))) {
-      e = chunk_f32_bwd(p, ptrs, ws, parts_bytes(p), &a.only, s);
-      if (e != hipSuccess) return e;
-    }
     const bool ok = with_width(p.Dk, [&](auto npt, auto lpr) {
       constexpr int NPT = decltype(npt)::value, LPR = decltype(lpr)::value;
       const dim3 block(Layout<NPT, LPR>::kThreads);
@@ -753,7 +727,7 @@ hipError_t launch_bwd(const Problem& p, const BwdPtrs& ptrs, void* ws, hipStream
   hipLaunchKernelGGL((rec_reduce_kernel<OutT>), dim3(static_cast<unsigned>((items + 7) / 8)), dim3(256), 0, s,
                      w.dq_part, w.dk_part, w.dg_part, w.db_part, ptrs.g, static_cast<OutT*>(ptrs.dq),
                      static_cast<OutT*>(ptrs.dk), ptrs.dg, static_cast<OutT*>(ptrs.dbeta), p.Hk, p.Hv, p.Dk, a.nblk,
-                     p.g_is_log, items, a.only);
+                     p.g_is_log, items);
   tr.mark();
   return hipGetLastError();
 }
@@ -773,19 +747,17 @@ size_t rec_ckpt_bytes(const Problem& p) {
 }
 
 size_t rec_workspace_bytes(const Problem& p) {
-  return parts_bytes(p) + (p.Dk > 256 ? rec_wide_scratch_bytes(p) : 0) + rec_flag_bytes(p);
+  const size_t nblk = row_blocks(p);
+  const size_t parts = (2 * size_t(p.BT) * p.Hv * nblk * p.Dk + 2 * size_t(p.BT) * p.Hv * nblk) * sizeof(float);
+  return parts + (p.Dk > 256 ? rec_wide_scratch_bytes(p) : 0);
 }
-
-// The word after the partials that the float32 chunk kernels raise (the recurrent kernels, which then write the
-// partials, read it meanwhile).
-size_t rec_flag_bytes(const Problem& p) { return chunk_f32_takes(p, kChunkF32FwdSteps, parts_bytes(p)) ? 16 : 0; }
 
 const char* const kRecFwdLaunches = "rec_fwd";
 const char* const kRecBwdLaunches = "rec_bwd,rec_reduce";
 
-hipError_t rec_fwd(const Problem& p, const FwdPtrs& a, void* ws, hipStream_t s, Tracer& tr) {
-  if (!p.in_bf16) return launch_fwd<float, float>(p, a, ws, s, tr);
-  return p.out_bf16 ? launch_fwd<bf16_t, bf16_t>(p, a, ws, s, tr) : launch_fwd<bf16_t, float>(p, a, ws, s, tr);
+hipError_t rec_fwd(const Problem& p, const FwdPtrs& a, void*, hipStream_t s, Tracer& tr) {
+  if (!p.in_bf16) return launch_fwd<float, float>(p, a, s, tr);
+  return p.out_bf16 ? launch_fwd<bf16_t, bf16_t>(p, a, s, tr) : launch_fwd<bf16_t, float>(p, a, s, tr);
 }
 
 hipError_t rec_bwd(const Problem& p, const BwdPtrs& a, void* ws, hipStream_t s, Tracer& tr) {
