@@ -27,7 +27,8 @@
  *   ckpt            qb_gdn_ckpt_bytes  float32        starts with the chunk-start states [NC, Hv, Dv, Dk]
  *   dq, dk          [B, T, Hk, Dk]     out dtype; dv [B, T, Hv, Dv] out dtype; dbeta [B, T, Hv] out dtype
  *   dg              [B, T, Hv]         float32
- * Pointers to q, k and ckpt must be 16-byte aligned, the others aligned to their element size.
+ * Pointers to q, k and ckpt must be 16-byte aligned, the others aligned to their element size. s_out may be s0's own
+ * buffer, and ds0 ds_out's.
  *
  * Semantics per value head and step (reference tests/gated_delta_ref.h:110-118):
  *   S~ = g_t S;  u = S~ k_t;  delta = beta_t (v_t - u);  S = S~ + delta k_t^T;  y_t = S q_t

@@ -193,7 +193,8 @@ def fwd_rows(desc, q, k, v, g, beta, s0, y, row_states, stream) -> None:
 
 
 def fwd(desc, q, k, v, g, beta, s0, y, s_out, ckpt, workspace, stream) -> None:
-    """desc, here and below, is a descriptor or a Plan. Pointers are ints (device addresses) or None; raises RuntimeError with the library's reason on failure."""
+    """desc, here and below, is a descriptor or a Plan. Pointers are ints (device addresses) or None; raises
+    RuntimeError with the library's reason on failure."""
     _call(load().qb_gdn_fwd, desc, q, k, v, g, beta, s0, y, s_out, ckpt, workspace, stream)
 
 

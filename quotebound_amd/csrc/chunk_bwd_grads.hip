@@ -202,10 +202,10 @@ __global__ __launch_bounds__(kThreads) void chunk_bwd_grads_kernel(ChunkArgs a) 
 
     for (int e = cur.e0; e < cur.e0 + cur.ne; ++e) {
       const int hv = hk * grp + e;
-      // The head whose tile and first block the end phase reads ahead, in two pieces in E1 and at the
-      // start of E2 (all of them in E2, whose products the waves then reach late, measured 154.3 against 153.1 us): the next in the group, the next item's first,
-      // or, for the block's last item, this head again (those reads are unused; they keep every path's loads the
-      // same, so the compiler's waits stay exact).
+      // The head whose tile and first block the end phase reads ahead, in two pieces, in E1 and at the start of E2 (all
+      // of them in E2, whose products the waves then reach late, measured 154.3 against 153.1 us): the next in the
+      // group, the next item's first, or, for the block's last item, this head again (those reads are unused; they keep
+      // every path's loads the same, so the compiler's waits stay exact).
       Item nx = cur;
       int nhv = hv;
       if (e + 1 < cur.e0 + cur.ne) {

@@ -27,9 +27,9 @@ struct ChunkArgs {
   void* dbeta;
   float* ds0;
   float* dsend;  // workspace: cotangent of each chunk's end state
-  // Workspace, with g given as the factor (null with no chunk slots): how many (chunk slot, value head) pairs hold a factor below kTinyFactor, then
-  // the pairs (slot * Hv + head), in no order. Cleared by the backward state pass, listed by the gradient kernel, taken
-  // up by chunk_dgfix.
+  // Workspace, with g given as the factor (null with no chunk slots): how many (chunk slot, value head) pairs hold a
+  // factor below kTinyFactor, then the pairs (slot * Hv + head), in no order. Cleared by the backward state pass, listed
+  // by the gradient kernel, taken up by chunk_dgfix.
   int* fix;
   float* dqk_part;  // workspace, short sequences: per (chunk slot, value head) dq and dk [64][128] float32, or null
   ChunkLayout lay;

@@ -1,9 +1,10 @@
 """The recurrent design on long float32 sequences against the oracle, on the GPU through the Python and the C entry
 points: lengths around whole chunks, one to three value heads per key head, one and several row blocks, ragged packed
 batches with empty sequences, the decay as log and as factor (negative and zero factors among them), values that are not
-finite, which must reach the outputs that they reach step by step and no others; and what the step-by-step order promises
-at any length: the float32 oracle's accuracy on keys that are nearly parallel, the same bits as the per-token states and as
-one-token calls, the same bits for a sequence alone and packed with others, and states updated in place.
+finite, which must reach the outputs that they reach step by step and no others; and what the step-by-step order
+promises at any length: the float32 oracle's accuracy on keys that are nearly parallel, the same bits as the per-token
+states and as one-token calls, the same bits for a sequence alone and packed with others, and states updated in place
+(these in the chunked design too).
 
 Tolerance, where no other is derived: 1e-5 of each output's largest value, the float32 criterion of the other tests.
 """
@@ -202,10 +203,11 @@ def test_accuracy_of_the_step_by_step_form(torch_dev, oracle, spread, beta, deca
     if spread is not None:
         inp["beta"], inp["g"] = np.full((1, T, 2), beta), np.full((1, T, 2), -decay)
     inp = _float32(inp)
-    exact, plain, got = oracle.fwd_bwd(inp, dtype=np.float64), oracle.fwd_bwd(inp, dtype=np.float32), _run(torch_dev, inp)
+    exact, plain = oracle.fwd_bwd(inp, dtype=np.float64), oracle.fwd_bwd(inp, dtype=np.float32)
+    got = _run(torch_dev, inp)
     err = lambda x, n: np.linalg.norm(x[n].astype(np.float64) - exact[n]) / np.linalg.norm(exact[n])  # noqa: E731
     errs = {n: (float(err(got, n)), float(err(plain, n))) for n in ("y", "s_out") + GRAD_NAMES}
-    print(f"spread {spread} beta {beta} decay {decay}: " + ", ".join(f"{n} {g:.1e} ({o:.1e})" for n, (g, o) in errs.items()))
+    print(f"spread {spread} beta {beta} decay {decay}:", {n: f"{g:.1e} ({o:.1e})" for n, (g, o) in errs.items()})
     assert all(g <= 2.0 * o for g, o in errs.values()), errs
 
 
@@ -254,16 +256,20 @@ def test_bits_of_a_packed_sequence(torch_dev):
         assert all(torch.equal(x[i:i + 1], z) for x, z in zip(states, s1)), (i, n)
 
 
-@pytest.mark.parametrize("where", [None, "v", "k", "beta", "s0", "dy", "ds_out"])
-def test_states_in_place(torch_dev, where):
+@pytest.mark.parametrize("design,where", [(_lib.RECURRENT, w) for w in (None, "v", "k", "beta", "s0", "dy", "ds_out")] +
+                         [(_lib.CHUNKED, None), (_lib.CHUNKED, "v")])
+def test_states_in_place(torch_dev, design, where):
     """Through the C entry points: s_out in s0's buffer and ds0 in ds_out's give what separate buffers give, with all
-    values finite and with a NaN in one of the inputs."""
+    values finite and with a NaN in one of the inputs. (The chunked design on bf16 activations.)"""
     torch = torch_dev
     T, Hk, Hv, Dv = 200, 2, 4, 64
     d = _device(torch, _float32(small_case(1, T, Hk, Hv, 128, Dv, seed=43)))
     if where:
         d[where].view(-1)[d[where].numel() // 2 + 17] = float("nan")
-    desc, keep = _lib.make_desc(1, T, Hk, Hv, 128, Dv, dtype=_lib.F32, design=_lib.RECURRENT)
+    if design == _lib.CHUNKED:
+        d.update({n: d[n].bfloat16() for n in ("q", "k", "v", "beta", "dy")})
+    dtype = _lib.F32 if design == _lib.RECURRENT else _lib.BF16
+    desc, keep = _lib.make_desc(1, T, Hk, Hv, 128, Dv, dtype=dtype, design=design)
     stream = torch.cuda.current_stream().cuda_stream
 
     def call(in_place):
